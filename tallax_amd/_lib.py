@@ -175,7 +175,7 @@ def require_cuda(*ts: torch.Tensor) -> None:
 
 def select_plan(rows: int, cols: int, dtype: int, k: int = 128, sample: bool = True) -> dict:
     """Work split of the selection kernels for a [rows, cols] input (host only).
-    A row is one whole-row workgroup (1024 threads, one segment), 2-4 equal
+    A row is one whole-row workgroup (1024 threads, one segment), 2-4
     whole-row parts (1024 threads, `segments` = parts) or 256-thread segments.
     Rows of several segments or parts finish in seg_merge64_pair_kernel (two
     lists) or seg_merge64_kernel for top-k with k <= 64 (no sampler), else in

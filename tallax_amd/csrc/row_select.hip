@@ -78,7 +78,7 @@ struct SelArgs {
   uint64_t* ws_lists;
   int lists_only;  // write the segment list even when a row is one segment
   int64_t col_offset;   // added to every column index of a written list (a vocabulary shard's first column)
-  int64_t part_cols;    // whole-row kernel on row parts: row r of the [np rows, cols / np] view adds (r % np) * part_cols
+  int64_t part_cols;    // whole-row kernel on row parts: part p of a row holds columns [p * part_cols, (p + 1) * part_cols)
   int nparts;
   int list_k;           // whole-row kernel: places of the row's (or part's) list that are read (64; 0: all 128)
   uint64_t* out_lists;  // merge kernel, lists_only: the merged list of each row, [rows][128]
@@ -690,6 +690,124 @@ __device__ __attribute__((noinline)) int tie_select(const uint4* base, int64_t s
   return wcnt;
 }
 
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) u32x4_t* GlobalVec;
+
+// Loaded in place of vectors past the end of a row: all-ones (negative NaNs)
+// never pass a filter and never raise a maximum.
+static __device__ u32x4_t g_dead_vec = {~0u, ~0u, ~0u, ~0u};
+
+// Class masks of a 16-byte vector for the ineligible classes: finfo.min
+// elements in bits 0-7, -inf in bits 8-15, NaN in bits 16-23 (all slots,
+// dead ones included).
+template <int DT>
+__device__ __forceinline__ uint32_t ineligible_masks(const uint4 v) {
+  constexpr bool kBF = DT == kBF16;
+  constexpr int VEC = ElemT<DT>::VEC;
+  constexpr uint32_t kMinB = kBF ? 0xFF7Fu : 0xFF7FFFFFu, kNegInfB = kBF ? 0xFF80u : 0xFF800000u;
+  constexpr uint32_t kAbs = kBF ? 0x7FFFu : 0x7FFFFFFFu, kInfAbs = kBF ? 0x7F80u : 0x7F800000u;
+  uint32_t m = 0;
+#pragma unroll
+  for (int q = 0; q < VEC; ++q) {
+    const uint32_t b = elem_bits<DT>(v, q);
+    m |= (b == kMinB ? 1u : 0u) << q;
+    m |= (b == kNegInfB ? 1u : 0u) << (8 + q);
+    m |= ((b & kAbs) > kInfAbs ? 1u : 0u) << (16 + q);
+  }
+  return m;
+}
+
+// The smallest (bits - finfo.min's bits) over the elements of a 16-byte
+// vector, wrapping in the element width: 0 when the vector holds finfo.min,
+// 1 when it holds -inf but not finfo.min, larger otherwise.
+template <int DT>
+__device__ __forceinline__ uint32_t min_offset_from_min(const uint4 v) {
+  if (DT == kBF16) {
+    const ushort2_t fm = __builtin_bit_cast(ushort2_t, 0xFF7FFF7Fu);
+    ushort2_t m = __builtin_bit_cast(ushort2_t, v.x) - fm;
+    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.y) - fm);
+    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.z) - fm);
+    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.w) - fm);
+    const uint32_t mm = __builtin_bit_cast(uint32_t, m);
+    const uint32_t lo = mm & 0xFFFFu, hi = mm >> 16;
+    return lo < hi ? lo : hi;
+  }
+  const uint32_t a = v.x - 0xFF7FFFFFu, b = v.y - 0xFF7FFFFFu, c = v.z - 0xFF7FFFFFu, d = v.w - 0xFF7FFFFFu;
+  const uint32_t ab = a < b ? a : b, cd = c < d ? c : d;
+  return ab < cd ? ab : cd;
+}
+
+// Rows with fewer than 128 eligible elements, all n of them candidates:
+// list[n..127] <- the first 128 - n ineligible elements in composite order --
+// the finfo.min elements, then -inf, then NaN, each class in index order --
+// and zeros where the row has fewer than 128 elements.  pmin / pinf: this
+// thread's vectors j (bit j) that may hold finfo.min or -inf, from the first
+// read (NaNs are not tracked: every vector may hold one); the vectors that
+// hold a class anywhere in the row are read again one at a time (vector j of
+// thread t at vector j * NT + t of row_base, nv vectors, the row's first
+// element at slot mis), in order, until the list is full.  A segment passes
+// its first vector as row_base and a negative mis, its first column.
+// tmp: 2 * NT / 64 words of LDS.  Out of line: a rare path kept out of the
+// kernel's hot code (the kernel's code size sets its instruction-cache
+// footprint).
+template <int DT, int V, int NT>
+__device__ __attribute__((noinline)) void fill_ineligible(const uint4* row_base, int nv, int mis, int cols, int n,
+                                                          uint32_t pmin, uint32_t pinf, uint64_t* list, int* red,
+                                                          uint32_t* tmp) {
+  constexpr bool kBF = DT == kBF16;
+  constexpr int VEC = ElemT<DT>::VEC, NW = NT / kWave;
+  constexpr uint32_t kMinKey = kBF ? 0x0080FFFFu : 0x00800000u;  // global keys of the three classes
+  constexpr uint32_t kNegInfKey = 0x007FFFFFu, kNaNKey = 1u;
+  const int tid = threadIdx.x;
+  const int w = tid / kWave, l = lane_id();
+  const GlobalVec gb = (GlobalVec)row_base;
+  const GlobalVec dead = (GlobalVec)(uintptr_t)&g_dead_vec;
+  pmin = wave_or_u32(pmin);
+  pinf = wave_or_u32(pinf);
+  if (l == 0) {
+    tmp[w] = pmin;
+    tmp[NW + w] = pinf;
+  }
+  __syncthreads();
+  pmin = 0;
+  pinf = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    pmin |= tmp[i];
+    pinf |= tmp[NW + i];
+  }
+  constexpr uint32_t kAll = (1u << V) - 1u;
+  int r = kMaxK - n, base = n;
+#pragma unroll 1
+  for (int c = 0; c < 3 && r > 0; ++c) {  // block-uniform
+    uint32_t pres = c == 0 ? pmin : (c == 1 ? pinf : kAll);
+    const uint32_t key = c == 0 ? kMinKey : (c == 1 ? kNegInfKey : kNaNKey);
+    while (pres && r > 0) {  // block-uniform: the vectors that may hold the class, in order
+      const int j = __builtin_ctz(pres);
+      pres &= pres - 1u;
+      const int v = j * NT + tid;
+      const u32x4_t x = *(v < nv ? gb + v : dead);
+      const int e0 = v * VEC - mis;
+      uint32_t m = (ineligible_masks<DT>(make_uint4(x.x, x.y, x.z, x.w)) >> (8 * c)) & 0xFFu;
+#pragma unroll
+      for (int q = 0; q < VEC; ++q)  // slots outside the row
+        m &= v < nv && (uint32_t)(e0 + q) < (uint32_t)cols ? ~0u : ~(1u << q);
+      int total;
+      int p = block_exscan<NW>(__popc(m), red, total);
+      while (m && p < r) {
+        const int q = __builtin_ctz(m);
+        m &= m - 1u;
+        list[base + p] = make_comp(key, (uint32_t)(e0 + q));
+        ++p;
+      }
+      const int took = total < r ? total : r;
+      base += took;
+      r -= took;
+    }
+  }
+  for (int i = base + tid; i < kMaxK; i += NT) list[i] = 0ull;
+}
+
 // ---------------------------------------------------------------------------
 // Kernel A: one workgroup per (segment, row).  The segment (MAXV 16-byte
 // vectors per thread) is loaded into registers with every load issued up
@@ -712,6 +830,7 @@ void seg_select_kernel(SelArgs a) {
   constexpr uint32_t kZeroKey = kBF ? 0x8000u : 0x80000000u;  // canonical key of +-0
   constexpr int32_t kPosInf = kBF ? 0x7F80 : 0x7F800000;      // +inf bits (signed / ordered view)
   constexpr int32_t kOrdNegInf = kBF ? -32641 : (int32_t)0x807FFFFFu;  // ordered view of -inf
+  constexpr uint32_t kFloor = kBF ? 0x0081u : 0x00800001u;  // smallest eligible canonical key
   __shared__ SegShared<C, NT> sh;
   __shared__ uint4 stage[kStage * NT];  // staged vectors, slot-major
   const int tid = threadIdx.x;
@@ -814,20 +933,33 @@ void seg_select_kernel(SelArgs a) {
   uint32_t L = sh.wl[0];
 #pragma unroll
   for (int i = 1; i < NW; ++i) L = sh.wl[i] < L ? sh.wl[i] : L;
-  const uint32_t thr = kBF ? L : (L > 1u ? L : 1u);  // candidates: live elements with canonical key >= thr
+  // candidates: eligible elements with canonical key >= thr.  A segment with
+  // fewer than k of them (constrained decoding: -inf but a few) takes the rest
+  // of its list by class (fill_ineligible) instead of collecting its -inf
+  // elements, which overflowed every region into the tie selection (sampler
+  // [67, 151937] f32, three rows in four masked: 65.5 -> 25.5 us).
+  const uint32_t thr = L > kFloor ? L : kFloor;
 
   // ---- flags: vectors whose maximum may reach thr ------------------------------
-  const bool nan_level = kBF ? thr == 0u : thr <= 1u;  // thr admits NaNs: every live vector
-  const bool pos_thr = !nan_level && thr > kZeroKey;   // positive threshold: signed view
+  const bool pos_thr = thr > kZeroKey;                 // positive threshold: signed view
   const int32_t st = (int32_t)(thr - kZeroKey);        // its bits, when positive
   uint32_t fl = 0;
   if (pos_thr) {
 #pragma unroll
     for (int j = 0; j < MAXV; ++j) fl |= (vec_smax<DT>(raw[j]) >= st ? 1u : 0u) << j;
   } else {
-    const int32_t ot = nan_level ? (int32_t)0x80000000u : (thr == kZeroKey ? -1 : (int32_t)(thr - kZeroKey));
+    const int32_t ot = thr == kZeroKey ? -1 : (int32_t)(thr - kZeroKey);
 #pragma unroll
     for (int j = 0; j < MAXV; ++j) fl |= (!vec_dead(j) && vec_omax<DT>(raw[j]) >= ot ? 1u : 0u) << j;
+  }
+  uint32_t pmin = 0, pinf = 0;  // thr at the floor: the vectors that may hold finfo.min / -inf
+  if (thr == kFloor) {          // block-uniform
+#pragma unroll
+    for (int j = 0; j < MAXV; ++j) {
+      const uint32_t o = min_offset_from_min<DT>(raw[j]);
+      pmin |= (o == 0u ? 1u : 0u) << j;
+      pinf |= (o <= 1u ? 1u : 0u) << j;
+    }
   }
   const int nfl = __popc(fl);
 
@@ -910,6 +1042,7 @@ void seg_select_kernel(SelArgs a) {
 
   // Filter pass; exact tie selection when a region overflows.  Control flow
   // is block-uniform.
+  int fill_from = kRun;  // candidates of a segment that has fewer than k
   {
     int wcnt = 0;
     rounds(wcnt);
@@ -918,6 +1051,12 @@ void seg_select_kernel(SelArgs a) {
     bool overflow = false;
 #pragma unroll
     for (int q = 0; q < NW; ++q) overflow |= sh.wc[q] > WCAP;
+    if (thr == kFloor && !overflow) {
+      int n = 0;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) n += sh.wc[q];
+      if (n < k) fill_from = n;
+    }
     if (overflow) {
       // its block sums order the reads of sh.wc above before the write below
       wcnt = tie_select<DT, MAXV, NT>(rv.base, s0, s1, lbase, live_lo, live_hi, gbase, k, reg, sh.red, stage);
@@ -928,6 +1067,10 @@ void seg_select_kernel(SelArgs a) {
 
   block_select(sh, (const int*)sh.wc);
   for (int i = tid; i < kRun; i += NT) sh.list64[i] = S::to_global(sh.list[i], seg_e0);
+  if (fill_from < kRun) {  // its first barriers order the writes above before its own
+    fill_ineligible<DT, MAXV, NT>(rv.base + s0, (int)(s1 - s0), -(int)seg_e0, (int)a.cols, fill_from, pmin, pinf,
+                                  sh.list64, sh.red, (uint32_t*)stage);
+  }
   __syncthreads();
   if (a.nseg == 1 && !a.lists_only) {
     finalize_row<DT, SAMPLE>(a, row, sh.list64, sh.samp_g, rp);
@@ -1047,7 +1190,7 @@ __global__ __launch_bounds__(kWave) void seg_merge64_pair_kernel(SelArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Kernel S (stream_select_kernel): a whole row (or one equal part of it) per
+// Kernel S (stream_select_kernel): a whole row (or one part of it) per
 // 1024-thread workgroup (16 waves, 4 per SIMD), V 16-byte vectors per thread
 // (V <= 19), vector j of thread t at row vector j * 1024 + t.
 //   1. Every load is issued up front.
@@ -1095,13 +1238,6 @@ struct StreamShared {
   int ncand;
   int ovf;                                 // a wave's staged vectors overflowed its region
 };
-
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-typedef const __attribute__((address_space(1))) u32x4_t* GlobalVec;
-
-// Loaded in place of vectors past the end of a row: all-ones (negative NaNs)
-// never pass a filter and never raise a maximum.
-static __device__ u32x4_t g_dead_vec = {~0u, ~0u, ~0u, ~0u};
 
 // lanes below this one in the wave
 __device__ __forceinline__ uint64_t lanes_below() {
@@ -1170,116 +1306,6 @@ __device__ __forceinline__ uint32_t pass_mask_ge(const uint4 vv, uint32_t thr) {
   return m;
 }
 
-// Class masks of a 16-byte vector for the ineligible classes: finfo.min
-// elements in bits 0-7, -inf in bits 8-15, NaN in bits 16-23 (all slots,
-// dead ones included).
-template <int DT>
-__device__ __forceinline__ uint32_t ineligible_masks(const uint4 v) {
-  constexpr bool kBF = DT == kBF16;
-  constexpr int VEC = ElemT<DT>::VEC;
-  constexpr uint32_t kMinB = kBF ? 0xFF7Fu : 0xFF7FFFFFu, kNegInfB = kBF ? 0xFF80u : 0xFF800000u;
-  constexpr uint32_t kAbs = kBF ? 0x7FFFu : 0x7FFFFFFFu, kInfAbs = kBF ? 0x7F80u : 0x7F800000u;
-  uint32_t m = 0;
-#pragma unroll
-  for (int q = 0; q < VEC; ++q) {
-    const uint32_t b = elem_bits<DT>(v, q);
-    m |= (b == kMinB ? 1u : 0u) << q;
-    m |= (b == kNegInfB ? 1u : 0u) << (8 + q);
-    m |= ((b & kAbs) > kInfAbs ? 1u : 0u) << (16 + q);
-  }
-  return m;
-}
-
-// The smallest (bits - finfo.min's bits) over the elements of a 16-byte
-// vector, wrapping in the element width: 0 when the vector holds finfo.min,
-// 1 when it holds -inf but not finfo.min, larger otherwise.
-template <int DT>
-__device__ __forceinline__ uint32_t min_offset_from_min(const uint4 v) {
-  if (DT == kBF16) {
-    const ushort2_t fm = __builtin_bit_cast(ushort2_t, 0xFF7FFF7Fu);
-    ushort2_t m = __builtin_bit_cast(ushort2_t, v.x) - fm;
-    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.y) - fm);
-    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.z) - fm);
-    m = __builtin_elementwise_min(m, __builtin_bit_cast(ushort2_t, v.w) - fm);
-    const uint32_t mm = __builtin_bit_cast(uint32_t, m);
-    const uint32_t lo = mm & 0xFFFFu, hi = mm >> 16;
-    return lo < hi ? lo : hi;
-  }
-  const uint32_t a = v.x - 0xFF7FFFFFu, b = v.y - 0xFF7FFFFFu, c = v.z - 0xFF7FFFFFu, d = v.w - 0xFF7FFFFFu;
-  const uint32_t ab = a < b ? a : b, cd = c < d ? c : d;
-  return ab < cd ? ab : cd;
-}
-
-// Rows with fewer than 128 eligible elements, all n of them candidates:
-// list[n..127] <- the first 128 - n ineligible elements in composite order --
-// the finfo.min elements, then -inf, then NaN, each class in index order --
-// and zeros where the row has fewer than 128 elements.  pmin / pinf: this
-// thread's vectors j (bit j) that may hold finfo.min or -inf, from the first
-// read (NaNs are not tracked: every vector may hold one); the vectors that
-// hold a class anywhere in the row are read again one at a time (vector j of
-// thread t at row vector j * kNTS + t of the aligned base, nv vectors, the
-// row's first element at slot mis), in order, until the list is full.
-// tmp: 2 * 16 words of LDS.  Out of line: a rare path kept out of the
-// kernel's hot code (the kernel's code size sets its instruction-cache
-// footprint).
-template <int DT, int V>
-__device__ __attribute__((noinline)) void fill_ineligible(const uint4* row_base, int nv, int mis, int cols, int n,
-                                                          uint32_t pmin, uint32_t pinf, uint64_t* list, int* red,
-                                                          uint32_t* tmp) {
-  constexpr bool kBF = DT == kBF16;
-  constexpr int VEC = ElemT<DT>::VEC, NW = kNTS / kWave;
-  constexpr uint32_t kMinKey = kBF ? 0x0080FFFFu : 0x00800000u;  // global keys of the three classes
-  constexpr uint32_t kNegInfKey = 0x007FFFFFu, kNaNKey = 1u;
-  const int tid = threadIdx.x;
-  const int w = tid / kWave, l = lane_id();
-  const GlobalVec gb = (GlobalVec)row_base;
-  const GlobalVec dead = (GlobalVec)(uintptr_t)&g_dead_vec;
-  pmin = wave_or_u32(pmin);
-  pinf = wave_or_u32(pinf);
-  if (l == 0) {
-    tmp[w] = pmin;
-    tmp[NW + w] = pinf;
-  }
-  __syncthreads();
-  pmin = 0;
-  pinf = 0;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    pmin |= tmp[i];
-    pinf |= tmp[NW + i];
-  }
-  constexpr uint32_t kAll = (1u << V) - 1u;
-  int r = kMaxK - n, base = n;
-#pragma unroll 1
-  for (int c = 0; c < 3 && r > 0; ++c) {  // block-uniform
-    uint32_t pres = c == 0 ? pmin : (c == 1 ? pinf : kAll);
-    const uint32_t key = c == 0 ? kMinKey : (c == 1 ? kNegInfKey : kNaNKey);
-    while (pres && r > 0) {  // block-uniform: the vectors that may hold the class, in order
-      const int j = __builtin_ctz(pres);
-      pres &= pres - 1u;
-      const int v = j * kNTS + tid;
-      const u32x4_t x = *(v < nv ? gb + v : dead);
-      const int e0 = v * VEC - mis;
-      uint32_t m = (ineligible_masks<DT>(make_uint4(x.x, x.y, x.z, x.w)) >> (8 * c)) & 0xFFu;
-#pragma unroll
-      for (int q = 0; q < VEC; ++q)  // slots outside the row
-        m &= (uint32_t)(e0 + q) < (uint32_t)cols ? ~0u : ~(1u << q);
-      int total;
-      int p = block_exscan<NW>(__popc(m), red, total);
-      while (m && p < r) {
-        const int q = __builtin_ctz(m);
-        m &= m - 1u;
-        list[base + p] = make_comp(key, (uint32_t)(e0 + q));
-        ++p;
-      }
-      const int took = total < r ? total : r;
-      base += took;
-      r -= took;
-    }
-  }
-  for (int i = base + tid; i < kMaxK; i += kNTS) list[i] = 0ull;
-}
-
 // Rows whose staged vectors or candidates overflow (heavy ties): tie_select
 // over the whole row, then the block's merge, into the sorted 128-entry list.
 // Out of line, like fill_ineligible.
@@ -1320,13 +1346,16 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   __shared__ uint4 stage[2 * kNTS];   // tie path
   const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
   const int64_t row = blockIdx.x;
-  const char* rowp = (const char*)a.x + (size_t)(row * a.cols) * ES;
+  // row parts (SAMPLE = false only): workgroup (row, part) of a two-dimensional
+  // grid; the row's last part may be shorter
+  const int64_t c0 = !SAMPLE && a.nparts > 1 ? (int64_t)blockIdx.y * a.part_cols : 0;
+  const int cols = (int)(!SAMPLE && a.nparts > 1 ? (a.cols - c0 < a.part_cols ? a.cols - c0 : a.part_cols) : a.cols);
+  const char* rowp = (const char*)a.x + (size_t)(row * a.cols + c0) * ES;
   const RowVec<ES> rv(rowp);
-  const int nv = (int)((a.cols + rv.mis + VEC - 1) / VEC);  // 1 <= nv <= kNTS * V (host plan)
+  const int nv = (cols + rv.mis + VEC - 1) / VEC;  // 1 <= nv <= kNTS * V (host plan)
   // list places the consumer reads: the bound guarantees kq elements, the
   // rank writes places below kq (the rest of the list is not read)
   const int kq = a.list_k == 64 ? 64 : kMaxK;
-  const int cols = (int)a.cols;
   const RowParams rp = load_row_params<SAMPLE>(a, row);
 
   if (tid == 0) ss.posted = 0;
@@ -1551,7 +1580,7 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   const bool fill = ss.ovf == 0 && n < kq && thr == kFloor;  // block-uniform
   // an overflowing staging region or more than kCandCap candidates: heavy ties
   const bool tie = !fill && (ss.ovf != 0 || n < kq || n > kCandCap);
-  if (fill) fill_ineligible<DT, V>(rv.base, nv, rv.mis, cols, n, pmin, pinf, sh.list64, sh.red, &ss.vsi[0][0]);
+  if (fill) fill_ineligible<DT, V, kNTS>(rv.base, nv, rv.mis, cols, n, pmin, pinf, sh.list64, sh.red, &ss.vsi[0][0]);
   if (tie) {
     stream_tie_path<DT, V>(rv.base, nv, rv.mis, cols, sh, stage);
   } else if (n > 0) {
@@ -1613,8 +1642,8 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   if (!a.lists_only) {
     finalize_row<DT, SAMPLE>(a, row, sh.list64, sh.samp_g, rp);
   } else {
-    uint64_t* dst = a.ws_lists + (size_t)row * kRun;
-    const uint64_t off = (uint64_t)(a.col_offset + (a.nparts > 1 ? (row % a.nparts) * a.part_cols : 0));
+    uint64_t* dst = a.ws_lists + (size_t)(row * gridDim.y + blockIdx.y) * kRun;
+    const uint64_t off = (uint64_t)(a.col_offset + c0);
     for (int i = tid; i < kq; i += kNTS) dst[i] = sh.list64[i] ? sh.list64[i] - off : 0ull;
   }
 }
@@ -1680,7 +1709,7 @@ struct Plan {
   int maxv;
   int nseg;
   int64_t vps;
-  int parts;  // > 1: whole-row kernel on that many equal parts of each row, then the merge
+  int parts;  // > 1: whole-row kernel on that many parts of each row, then the merge
 };
 
 // Work split.  A row of nv 16-byte vectors is handled either
@@ -1694,7 +1723,7 @@ struct Plan {
 //     16.7 -> 11.8; 19 vectors per thread for the 151936-wide bf16
 //     vocabulary: sampler [64, 151936] 20.5 -> 12.7, [256, 151936] 25.2 ->
 //     17.8; no shape slower); or
-//   * as 2-4 equal parts of at most 19 vectors per thread when the row
+//   * as 2-4 parts of at most 19 vectors per thread when the row
 //     divides and rows x parts <= kPartsMaxBlocks: the whole-row kernel
 //     writes each part's top-128 list (rows of the [parts x rows, cols /
 //     parts] view, column offsets added back), then the per-row merge
@@ -1782,24 +1811,24 @@ static void launch_a(const SelArgs& a, hipStream_t s) {
 
 template <int DT, bool SAMPLE>
 static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const char* what) {
-  // parts: the whole-row kernel writes each part's list (no sampling; its
-  // rows are the [np rows, cols / np] view), the merge kernel finishes the row
+  // parts: the whole-row kernel writes each part's list (no sampling), the
+  // merge kernel finishes the row
   SelArgs h = a0;
   // top-k with k <= 64 reads the first 64 places of a row's (or a part's) list
   if (!SAMPLE && !a0.lists_only && a0.k <= kWave) h.list_k = kWave;
   if (p.parts > 1) {
-    h.rows = a0.rows * p.parts;
-    h.cols = a0.cols / p.parts;
     h.nseg = 1;
     h.lists_only = 1;
-    h.part_cols = h.cols;
+    h.part_cols = a0.cols / p.parts;
     h.nparts = p.parts;
-
   }
   const SelArgs& a = h;
   if (p.nt == kNTS && p.parts > 1) {
-    const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0;
-    const dim3 g((unsigned)a.rows), b(kNTS);
+    // every row and every part starts 16-byte aligned and fills its last vector
+    // (the row's last part too: cols and part_cols both are whole vectors)
+    const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0 ||
+                      (a.part_cols * ElemT<DT>::ES) % 16 != 0;
+    const dim3 g((unsigned)a.rows, (unsigned)p.parts), b(kNTS);
     if (p.maxv == 19) {
       if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true>), g, b, 0, s, a);
       else hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, false>), g, b, 0, s, a);

@@ -1,0 +1,47 @@
+"""Rows too long for one workgroup: segments with fewer than 128 eligible
+values, and parts of rows that do not divide, against the oracle bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import bits, from_dev_vals, host_values, to_dev
+from oracle import tallax_oracle as O
+from test_gpu_select import _make
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(gpu, rows, cols, k, dtype, kind, threads, segments=None):
+    from tallax_amd import _lib, sampling, tax
+    print(f"split rows={rows} cols={cols} k={k} {dtype} {kind}", flush=True)
+    x = _make(rows, cols, kind, seed=rows * 31 + cols)
+    xd, xv = to_dev(x, dtype, gpu), host_values(x, dtype)
+    plan = _lib.select_plan(rows, cols, _lib.dtype_code(xd))
+    assert plan["threads"] == threads and (segments is None or plan["segments"] == segments), plan
+    vals, idx = tax.top_k(xd, k)
+    ov, oi = O.top_k(xv, k, dtype)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    assert np.array_equal(bits(from_dev_vals(vals)), bits(ov))
+    rng = np.random.default_rng(cols)
+    temp = rng.uniform(0.5, 1.5, rows).astype(np.float32)
+    topk = rng.integers(1, 200, rows).astype(np.int32)
+    topp = rng.uniform(0.7, 1.0, rows).astype(np.float32)
+    meta = sampling.SamplingMetadata(*(torch.from_numpy(a).to(gpu) for a in (topk, topp, temp)))
+    tok = sampling.sample((3, 77), xd, meta).cpu().numpy()
+    assert np.array_equal(tok, O.sample((3, 77), xv, topk, topp, temp, dtype=dtype))
+
+
+# rows of segments: every class of ineligible value fills the list's end, in
+# rows whose masked stretches span several segments, aligned or not, and in
+# the row's short last segment
+@pytest.mark.parametrize("rows,cols,k,dtype,kind", [
+    (8, 200003, 128, "f32", "masked_mix"),
+    (8, 200003, 64, "f32", "masked_mix"),
+    (16, 311299, 128, "bf16", "masked_mix"),
+    (9, 155653, 100, "bf16", "masked_mix"),
+    (4, 81931, 128, "f32", "nan_heavy"),
+    (5, 200003, 128, "f32", "masked5"),
+    (6, 155653, 128, "bf16", "special"),
+])
+def test_segments_with_few_eligible(gpu, rows, cols, k, dtype, kind):
+    _check(gpu, rows, cols, k, dtype, kind, 256)
