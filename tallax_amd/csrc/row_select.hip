@@ -63,6 +63,8 @@ constexpr int kRun = 128;                  // list length handed between kernels
 constexpr int kMaxSeg = 32;
 constexpr int kTargetBlocks = 1024;        // ~4 workgroups per CU on 256 CUs
 constexpr int kPartsMaxBlocks = 512;       // whole-row parts: two rounds of one workgroup per CU at most
+constexpr int kUnevenMinBlocks = 128;      // parts of a row that does not divide: one round that fills
+constexpr int kUnevenMaxBlocks = 256;      // at least half of the CUs (plan_rows)
 
 struct SelArgs {
   const void* x;
@@ -1730,13 +1732,30 @@ struct Plan {
 //     (config 3, [128, 151936] f32: 21.50 -> 20.05 us; f32 sampler
 //     [64, 128256] 19.5 -> 15.7, [64, 201088] 26.9 -> 17.2; at more blocks
 //     the segments win: [256, 201088] 46.5 against 50.4, [512, 151936]
-//     top-k 55.1 against 62.6); or
+//     top-k 55.1 against 62.6); rows that do not divide take parts of whole
+//     vectors, the last one shorter, where 128 to 256 part workgroups make
+//     one round over at least half of the CUs (f32, segments -> parts: sampler
+//     [64, 151937] 24.3 -> 19.3 us, [128, 151937] 26.7 -> 23.1, [64, 220001]
+//     28.8 -> 21.0; top-k k = 50 [64, 151937] 18.3 -> 17.0; bf16 sampler
+//     [48, 220001] 22.9 -> 17.8, [128, 220001] masked 33.0 -> 26.1).  Fewer rows
+//     do better in segments, which spread each row over more CUs (top-k
+//     [16, 151937] 12.2 against 15.6 us, masked sampler [32, 220001] 21.2
+//     against 23.3), and so does a second round ([128, 220001] f32 sampler
+//     34.0 against 36.0); or
 //   * in segments of 256 x MAXV vectors, MAXV in {4, 8, 16, 19}: the largest that
 //     still gives ~4 workgroups per CU over the launch, then a per-row merge;
 //     where 16 gives more than one residency round (4 workgroups per CU,
 //     kTargetBlocks) and 19 gives exactly one, MAXV = 19 (config 3: 8
 //     segments of 19 vectors per thread instead of 10 of 16, measured
 //     22.03 -> 21.45 us).
+// Columns per part: equal parts when the row divides, else whole vectors with a
+// shorter last part.
+static int64_t part_cols_of(int64_t cols, int np, int vec) {
+  if (cols % np == 0) return cols / np;
+  const int64_t per = (cols + np - 1) / np;
+  return (per + vec - 1) / vec * vec;
+}
+
 static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
   const int vec = dt == kF32 ? 4 : 8;
   const int64_t nv = (cols + 2 * (vec - 1)) / vec;  // covers any row misalignment
@@ -1751,9 +1770,12 @@ static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
     p->vps = (int64_t)kNTS * maxv;
     return kOk;
   }
-  for (int np = 2; np <= 4 && rows * np <= kPartsMaxBlocks; ++np) {  // equal whole-row parts
-    if (cols % np) continue;
-    const int64_t nvh = (cols / np + 2 * (vec - 1)) / vec;
+  for (int o = 0; o < 6; ++o) {  // whole-row parts, equal ones first
+    const int np = 2 + o % 3;
+    if (o < 3 ? cols % np != 0 || rows * np > kPartsMaxBlocks
+              : rows * np < kUnevenMinBlocks || rows * np > kUnevenMaxBlocks)
+      continue;
+    const int64_t nvh = (part_cols_of(cols, np, vec) + 2 * (vec - 1)) / vec;
     if (nvh <= (int64_t)kNTS * 19) {
       p->nt = kNTS;
       p->maxv = nvh > (int64_t)kNTS * 16 ? 19 : 16;
@@ -1819,7 +1841,7 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
   if (p.parts > 1) {
     h.nseg = 1;
     h.lists_only = 1;
-    h.part_cols = a0.cols / p.parts;
+    h.part_cols = part_cols_of(a0.cols, p.parts, ElemT<DT>::VEC);
     h.nparts = p.parts;
   }
   const SelArgs& a = h;

@@ -45,3 +45,19 @@ def _check(gpu, rows, cols, k, dtype, kind, threads, segments=None):
 ])
 def test_segments_with_few_eligible(gpu, rows, cols, k, dtype, kind):
     _check(gpu, rows, cols, k, dtype, kind, 256)
+
+
+# rows that do not divide: parts of whole vectors with a shorter last one, at
+# both ends of the 128..256 part workgroups, misaligned rows among them
+@pytest.mark.parametrize("rows,cols,k,dtype,kind,parts", [
+    (64, 77827, 128, "f32", "masked_mix", 2),    # the shortest such row
+    (64, 151937, 50, "f32", "normal", 2),
+    (128, 155623, 128, "f32", "masked_mix", 2),  # parts of 19 vectors per thread
+    (44, 220001, 64, "f32", "masked_mix", 3),
+    (32, 311233, 100, "f32", "special", 4),
+    (64, 155653, 64, "bf16", "masked_mix", 2),
+    (70, 200003, 128, "bf16", "tieblock", 2),
+    (43, 400003, 50, "bf16", "normal", 3),
+])
+def test_uneven_parts(gpu, rows, cols, k, dtype, kind, parts):
+    _check(gpu, rows, cols, k, dtype, kind, 1024, parts)
