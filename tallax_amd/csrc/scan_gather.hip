@@ -15,6 +15,8 @@
 //     in that order; int32: wrapping adds).
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "tallax_hip.h"
 #include "tx_common.h"
 #include "tx_host.h"
@@ -211,15 +213,65 @@ __device__ __forceinline__ T readlane_t(T v, int src) {
   return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
 }
 
-// Axis 1, one workgroup per row, 16 waves; wave w scans tiles w, w + 16, ...
-// of a chunk of 64 tiles held in registers (two elements per lane per tile:
-// tile position p = h * 64 + lane).  The next chunk's loads are issued before
-// this chunk's carries are chained, and wave 0 chains the 64 tile totals with
-// readlanes (one dependent add per tile).
+// Eight consecutive elements of a row as the scan takes them: c[h] = element
+// e + h, reversed e + 7 - h; elements at or past n read as 0.  Rows need only
+// their elements' own alignment: the 16-byte accesses are 4-byte aligned.
+struct __attribute__((packed, aligned(4))) Quad4 {
+  uint32_t v[4];
+};
+template <typename T>
+__device__ __forceinline__ void load8(const T* row, int64_t e, int64_t n, int reverse, T (&c)[8]) {
+  uint32_t u[8];
+  if (e + 8 <= n) {
+    const Quad4 a = *(const Quad4*)(row + e), b = *(const Quad4*)(row + e + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      u[i] = a.v[i];
+      u[4 + i] = b.v[i];
+    }
+  } else {  // the row's end: clamped loads, no branch per element
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = ((const uint32_t*)row)[e + i < n ? e + i : n - 1];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = e + i < n ? u[i] : 0u;
+  }
+#pragma unroll
+  for (int h = 0; h < 8; ++h) c[h] = __builtin_bit_cast(T, reverse ? u[7 - h] : u[h]);
+}
+// The same elements back; `keep_last`: the last scan position (h = 7) is not
+// written.
+template <typename T>
+__device__ __forceinline__ void store8(T* row, int64_t e, int64_t n, int reverse, const T (&c)[8], bool keep_last) {
+  uint32_t u[8];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) u[h] = __builtin_bit_cast(uint32_t, reverse ? c[7 - h] : c[h]);
+  if (e + 8 <= n && !keep_last) {
+    Quad4 a, b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a.v[i] = u[i];
+      b.v[i] = u[4 + i];
+    }
+    *(Quad4*)(row + e) = a;
+    *(Quad4*)(row + e + 4) = b;
+  } else {
+    const int skip = keep_last ? (reverse ? 0 : 7) : 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i != skip && e + i < n) ((uint32_t*)row)[e + i] = u[i];
+  }
+}
+
+// Axis 1, one workgroup per row, 16 waves; wave w scans tiles 4 w .. 4 w + 3 of
+// a chunk of 64 tiles held in registers, one per 16-lane row (hs_scan128_rows).
+// The next chunk's loads are issued before this chunk's carries are chained,
+// and wave 0 chains the 64 tile totals with readlanes (one dependent add per
+// tile).  [2048, 8192] f32 50.8 -> 36 us, [256, 128256] 85.4 -> 81.6 against the
+// scan through the LDS crossbar; three chunks of loads in flight were slower
+// ([2048, 8192] 45.5, [512, 32768] 41.9 -> 50.3).
 constexpr int kScanNT = 1024;
 constexpr int kScanNW = kScanNT / kWave;
-constexpr int kTPW = 4;                        // tiles per wave per chunk
-constexpr int kChunkTiles = kScanNW * kTPW;    // 64 tiles = 8192 elements
+constexpr int kChunkTiles = kScanNW * 4;       // 64 tiles = 8192 elements
 static_assert(kChunkTiles == kWave, "one tile total per lane of wave 0");
 
 template <typename T>
@@ -230,33 +282,23 @@ __global__ __launch_bounds__(kScanNT) void cumsum_rows_kernel(const T* __restric
   __shared__ T run_sh;
   const int64_t r = blockIdx.x;
   const int w = threadIdx.x / kWave, l = lane_id();
+  const int tc = threadIdx.x / 16;                 // this lane's tile of the chunk
   const int64_t pcols = (cols + 127) / 128 * 128;  // padded length
   const int64_t ntiles = pcols / 128;
   const T* xr = x + r * cols;
   T* orow = out + r * cols;
-  auto load_chunk = [&](int64_t t0, T (&c)[kTPW][2]) {
-#pragma unroll
-    for (int i = 0; i < kTPW; ++i) {
-      const int64_t t = t0 + w + (int64_t)i * kScanNW;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t q = t * 128 + h * kWave + l;
-        const int64_t e = reverse ? pcols - 1 - q : q;
-        c[i][h] = (t < ntiles && e < cols) ? xr[e] : (T)0;
-      }
-    }
+  auto elem = [&](int64_t t0) -> int64_t {  // first of this lane's eight elements
+    const int64_t q = (t0 + tc) * 128 + 8 * (l & 15);
+    return reverse ? pcols - 8 - q : q;
   };
-  T c[kTPW][2];
-  load_chunk(0, c);
+  T c[8];
+  load8(xr, tc < ntiles ? elem(0) : cols, cols, reverse, c);
   T run = (T)0;
   for (int64_t t0 = 0; t0 < ntiles; t0 += kChunkTiles) {
-#pragma unroll
-    for (int i = 0; i < kTPW; ++i) {
-      hs_scan128(c[i], l);
-      if (l == kWave - 1) tsum[w + i * kScanNW] = c[i][1];
-    }
-    T nx[kTPW][2];
-    load_chunk(t0 + kChunkTiles, nx);
+    hs_scan128_rows(c);
+    if ((l & 15) == 15) tsum[tc] = c[7];
+    T nx[8];
+    load8(xr, t0 + kChunkTiles + tc < ntiles ? elem(t0 + kChunkTiles) : cols, cols, reverse, nx);
     lds_barrier();
     // sequential running total over the chunk's tiles (reference order)
     if (w == 0) {
@@ -272,32 +314,24 @@ __global__ __launch_bounds__(kScanNT) void cumsum_rows_kernel(const T* __restric
       if (l == 0) run_sh = acc;
     }
     lds_barrier();
+    if (t0 + tc < ntiles) {
+      const T cy = carry[tc];
+      if (t0 + tc > 0) {
 #pragma unroll
-    for (int i = 0; i < kTPW; ++i) {
-      const int64_t t = t0 + w + (int64_t)i * kScanNW;
-      if (t >= ntiles) continue;
-      const T cy = carry[w + i * kScanNW];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t q = t * 128 + h * kWave + l;
-        const int64_t e = reverse ? pcols - 1 - q : q;
-        const T v = t == 0 ? c[i][h] : add_in_order(c[i][h], cy);
-        if (e < cols) orow[e] = v;
+        for (int h = 0; h < 8; ++h) c[h] = add_in_order(c[h], cy);
       }
+      store8(orow, elem(t0), cols, reverse, c, false);
     }
     run = run_sh;
 #pragma unroll
-    for (int i = 0; i < kTPW; ++i) {
-      c[i][0] = nx[i][0];
-      c[i][1] = nx[i][1];
-    }
+    for (int h = 0; h < 8; ++h) c[h] = nx[h];
     // no third barrier: the next writes of tsum, carry and run_sh follow the
     // next chunk's first barrier, which every wave reaches after its reads
   }
 }
 
-// Axis 1, any number of rows, in three launches (each tile scanned by one
-// wave, so the chip fills whatever the row count):
+// Axis 1, any number of rows, in three launches (four tiles per wave at a
+// time, so the chip fills whatever the row count):
 //   FINAL = false: scan tiles 0 .. ntiles - 2 of every row and stage each
 //                  tile's total in `out` (tile_stage_pos);
 //   cumsum_chain_kernel: chain the staged totals and store the final values
@@ -305,9 +339,16 @@ __global__ __launch_bounds__(kScanNT) void cumsum_rows_kernel(const T* __restric
 //   FINAL = true:  scan every tile again and add the carry (the previous
 //                  tile's final last position); positions already final are
 //                  not written, staged totals are overwritten.
+// Bound by HBM (x read twice, out written once): [64, 128257] f32 15.8 -> 9.2 us
+// for the first pass, 19.4 -> 16.6 for the last (half a wave per tile, 4-byte
+// loads and LDS-crossbar scans before).
 constexpr int kTileWaves = 4;      // waves per workgroup
-constexpr int kTilesPerWave = 4;   // tiles per wave, loads issued together
-template <typename T, bool FINAL>
+// G groups of four tiles per wave, loads issued together: 4, or 1 where 4 would
+// leave the chip short of waves (below 65536 tiles, 4096 waves: [3000, 333]
+// 14.5 us against 18.6 with 4, [1024, 2048] 16.2 against 17.9).
+constexpr int kTileGroups = 4;
+constexpr int64_t kTileTasksMany = 65536;
+template <typename T, bool FINAL, int G>
 __global__ __launch_bounds__(kTileWaves * kWave) void cumsum_row_tiles_kernel(const T* __restrict__ x, int64_t rows,
                                                                               int64_t cols, int64_t ntiles,
                                                                               int reverse, T* __restrict__ out) {
@@ -315,42 +356,49 @@ __global__ __launch_bounds__(kTileWaves * kWave) void cumsum_row_tiles_kernel(co
   const int64_t per_row = FINAL ? ntiles : ntiles - 1;
   const int64_t ntask = rows * per_row;
   const int64_t pcols = ntiles * 128;
-  const int64_t g0 = ((int64_t)blockIdx.x * kTileWaves + threadIdx.x / kWave) * kTilesPerWave;
-  T c[kTilesPerWave][2];
-  T cy[kTilesPerWave];
-  int64_t rr[kTilesPerWave], tt[kTilesPerWave];
+  const int64_t g0 = ((int64_t)blockIdx.x * kTileWaves + threadIdx.x / kWave) * (4 * G);
+  if (g0 >= ntask) return;
+  // the wave's first tile (one scalar division), then each lane's
+  const int64_t r0 = ntask <= 0xFFFFFFFFll ? (int64_t)((uint32_t)g0 / (uint32_t)per_row) : g0 / per_row;
+  const int64_t m0 = g0 - r0 * per_row;
+  T c[G][8];
+  T cy[G];
+  int64_t rr[G], tt[G], ee[G];
 #pragma unroll
-  for (int i = 0; i < kTilesPerWave; ++i) {
-    const int64_t g = g0 + i;
-    rr[i] = g < ntask ? g / per_row : -1;
-    tt[i] = g < ntask ? g - rr[i] * per_row : 0;
-    const T* xr = x + rr[i] * cols;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t q = tt[i] * 128 + h * kWave + l;
-      const int64_t e = reverse ? pcols - 1 - q : q;
-      c[i][h] = (rr[i] >= 0 && e < cols) ? xr[e] : (T)0;
+  for (int i = 0; i < G; ++i) {
+    const int d = 4 * i + (l >> 4);
+    int64_t r = r0, t = m0 + d;
+    if (t >= per_row) {  // at most (4 * G) - 1 past the end of row r0
+      const uint32_t over = (uint32_t)(t - per_row);
+      const uint32_t pr = per_row > (4 * G) ? (uint32_t)(4 * G) : (uint32_t)per_row;
+      const uint32_t k = over / pr;
+      r += 1 + k;
+      t = over - k * pr;
     }
-    cy[i] = (FINAL && rr[i] >= 0 && tt[i] > 0) ? out[rr[i] * cols + tile_last_pos(tt[i] - 1, 128, pcols, reverse)]
-                                               : (T)0;
+    const bool in = g0 + d < ntask;
+    if (!in) r = 0;
+    const int64_t q = t * 128 + 8 * (l & 15);
+    rr[i] = in ? r : -1;
+    tt[i] = t;
+    ee[i] = reverse ? pcols - 8 - q : q;
+    load8(x + r * cols, in ? ee[i] : cols, cols, reverse, c[i]);
+    cy[i] = (FINAL && in && t > 0) ? out[r * cols + tile_last_pos(t - 1, 128, pcols, reverse)] : (T)0;
   }
 #pragma unroll
-  for (int i = 0; i < kTilesPerWave; ++i) {
-    hs_scan128(c[i], l);
+  for (int i = 0; i < G; ++i) {
+    hs_scan128_rows(c[i]);
     if (rr[i] < 0) continue;
     T* orow = out + rr[i] * cols;
     if (!FINAL) {
-      if (l == kWave - 1) orow[tile_stage_pos(tt[i], 128, reverse)] = c[i][1];
+      if ((l & 15) == 15) orow[tile_stage_pos(tt[i], 128, reverse)] = c[i][7];
       continue;
     }
-    const bool last_final = tt[i] < ntiles - 1;  // the last position already holds its final value
+    if (tt[i] > 0) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t q = tt[i] * 128 + h * kWave + l;
-      const int64_t e = reverse ? pcols - 1 - q : q;
-      const T v = tt[i] == 0 ? c[i][h] : add_in_order(c[i][h], cy[i]);
-      if (e < cols && !(last_final && h == 1 && l == kWave - 1)) orow[e] = v;
+      for (int h = 0; h < 8; ++h) c[i][h] = add_in_order(c[i][h], cy[i]);
     }
+    // the last position of a tile with a successor already holds its final value
+    store8(orow, ee[i], cols, reverse, c[i], (l & 15) == 15 && tt[i] < ntiles - 1);
   }
 }
 
@@ -546,13 +594,20 @@ static unsigned grid_for(int64_t total) {
 }
 
 
-// One workgroup per row pays off for >= 256 rows of >= 64 tiles (measured on
-// f32: [256, 128256] 84 us against 114 us in three launches, [512, 32768]
-// 46 against 63, [2048, 8192] 50 against 62); fewer rows leave CUs idle and
-// shorter rows leave its waves idle ([4096, 4096] 83 against 63 us,
-// [1024, 2048] 21.3 against 18.8), so those take the three launches.
-constexpr int64_t kRowKernelMinRows = 256;
-constexpr int64_t kRowKernelMinTiles = 64;
+// One launch with a workgroup per row, or three over tiles.  The row kernel costs
+// about 2 + 5 us per round of 256 rows and chunk of 64 tiles, a partial round
+// or chunk as much as a whole one; the three launches about 10 us + 2.8 us per
+// million elements (f32 and int32, row kernel / three launches in us:
+// [256, 8192] 6.7 / 16.4, [256, 128256] 82 / 102, [2048, 8192] 37 / 50,
+// [512, 32768] 42 / 52; [300, 100003] 125 / 93, [3230, 8552] 123 / 85,
+// [300, 20001] 31 / 27, [4096, 4096] 82 / 50, [1, 333] 4.5 / 10.0, [16, 8192]
+// 5.1 / 11.2, [64, 16384] 11.5 / 13.7).  Rows of one tile need one tile launch
+// (3.0 us against 4.4 for [1, 100]).
+static bool cumsum_row_route(int64_t rows, int64_t cols) {
+  const double rounds = (double)((rows + 255) / 256);
+  const double chunks = (double)((cols + 128 * kChunkTiles - 1) / (128 * kChunkTiles));
+  return cols > 128 && rows <= 2147483647 && 2.0 + 5.0 * rounds * chunks <= 10.0 + 2.8e-6 * (double)rows * (double)cols;
+}
 
 // cumsum as tile totals -> sequential chain over them -> rescan plus carry
 // (one launch when every line is a single tile).
@@ -563,19 +618,28 @@ static void cumsum_three_launch(const T* x, int64_t rows, int64_t cols, int axis
   const int64_t len = axis == 1 ? cols : rows;
   const int64_t nlines = axis == 1 ? rows : cols;
   const int64_t ntiles = (len + ts - 1) / ts;
+  const bool many = ntiles * nlines >= kTileTasksMany;
   auto tile_grid = [&](int64_t per_line) -> unsigned {
     const int64_t tasks = per_line * nlines;
-    const int64_t per_block = axis == 1 ? (int64_t)kTileWaves * kTilesPerWave : 256;
+    const int64_t per_block = axis == 1 ? (int64_t)kTileWaves * 4 * (many ? kTileGroups : 1) : 256;
     const int64_t b = (tasks + per_block - 1) / per_block;
     return (unsigned)(b > 2147483647 ? 2147483647 : b);
   };
-  const unsigned tile_nt = axis == 1 ? kTileWaves * kWave : 256;
-  if (ntiles > 1) {
-    if (axis == 1)
-      hipLaunchKernelGGL((cumsum_row_tiles_kernel<T, false>), dim3(tile_grid(ntiles - 1)), dim3(tile_nt), 0, stream,
+  // the tile scans of axis 1: G tile groups per wave
+  auto row_tiles = [&](auto final_pass, unsigned grid) {
+    constexpr bool F = decltype(final_pass)::value;
+    if (many)
+      hipLaunchKernelGGL((cumsum_row_tiles_kernel<T, F, kTileGroups>), dim3(grid), dim3(kTileWaves * kWave), 0, stream,
                          x, rows, cols, ntiles, reverse, out);
     else
-      hipLaunchKernelGGL((cumsum_col_tiles_kernel<T, false>), dim3(tile_grid(ntiles - 1)), dim3(tile_nt), 0, stream,
+      hipLaunchKernelGGL((cumsum_row_tiles_kernel<T, F, 1>), dim3(grid), dim3(kTileWaves * kWave), 0, stream, x, rows,
+                         cols, ntiles, reverse, out);
+  };
+  if (ntiles > 1) {
+    if (axis == 1)
+      row_tiles(std::false_type{}, tile_grid(ntiles - 1));
+    else
+      hipLaunchKernelGGL((cumsum_col_tiles_kernel<T, false>), dim3(tile_grid(ntiles - 1)), dim3(256), 0, stream,
                          x, rows, cols, ntiles, reverse, out);
     // lines per chain workgroup: enough workgroups to spread the loads, the
     // lanes of wave 0 chaining their lines side by side
@@ -587,10 +651,9 @@ static void cumsum_three_launch(const T* x, int64_t rows, int64_t cols, int axis
                        ntiles - 1, gl, axis == 1 ? 1 : 0);
   }
   if (axis == 1)
-    hipLaunchKernelGGL((cumsum_row_tiles_kernel<T, true>), dim3(tile_grid(ntiles)), dim3(tile_nt), 0, stream, x,
-                       rows, cols, ntiles, reverse, out);
+    row_tiles(std::true_type{}, tile_grid(ntiles));
   else
-    hipLaunchKernelGGL((cumsum_col_tiles_kernel<T, true>), dim3(tile_grid(ntiles)), dim3(tile_nt), 0, stream, x,
+    hipLaunchKernelGGL((cumsum_col_tiles_kernel<T, true>), dim3(tile_grid(ntiles)), dim3(256), 0, stream, x,
                        rows, cols, ntiles, reverse, out);
 }
 
@@ -695,8 +758,7 @@ int tallax_cumsum(const void* x, int dtype, int64_t rows, int64_t cols, int axis
       hipLaunchKernelGGL((cumsum_narrow_rows_kernel<int32_t, kNarrowCols>), dim3(grid), dim3(256), 0, stream,
                          (const int32_t*)x, rows, (int)cols, reverse, (int32_t*)out);
   } else if (axis == 1) {
-    const int64_t ntiles = (cols + 127) / 128;
-    if (rows >= kRowKernelMinRows && ntiles >= kRowKernelMinTiles && rows <= 2147483647) {
+    if (cumsum_row_route(rows, cols)) {
       if (dtype == kF32)
         hipLaunchKernelGGL(cumsum_rows_kernel<float>, dim3((unsigned)rows), dim3(kScanNT), 0, stream,
                            (const float*)x, cols, reverse, (float*)out);

@@ -80,6 +80,42 @@ __device__ __forceinline__ int block_sum(int v, int* red) {
   return t;
 }
 
+// Value of the lane d below in the same 16-lane DPP row, +0 below the row's
+// start (row_shr:d, zero fill); d in {1, 2, 4, 8}, constant after unrolling.
+template <typename T>
+__device__ __forceinline__ T row_up_or_zero(T v, int d) {
+  const int x = __builtin_bit_cast(int, v);
+  switch (d) {
+    case 1: return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true));
+    case 2: return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true));
+    case 4: return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true));
+    default: return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true));
+  }
+}
+
+// Hillis-Steele inclusive scans of four 128-position tiles per wave, one per
+// 16-lane DPP row: position p = 8 * (lane & 15) + h.  Every step adds position
+// p - s, or +0 below position 0, in one VALU add (a DPP operand where the
+// partner is in another lane): 56 adds for four tiles, no LDS crossbar.  The
+// layout of hs_scan128 needs 18 ds_bpermute and about 60 VALU instructions per
+// tile (cumsum [64, 128257] f32, three launches: 48.5 -> 38.8 us).
+template <typename T>
+__device__ __forceinline__ void hs_scan128_rows(T (&c)[8]) {
+#pragma unroll
+  for (int s = 1; s < 128; s <<= 1) {
+    T n[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+      if (s < 8)
+        n[h] = add_in_order(c[h], h >= s ? c[h - s] : row_up_or_zero(c[h - s + 8 < 8 ? h - s + 8 : 0], 1));
+      else
+        n[h] = add_in_order(c[h], row_up_or_zero(c[h], s / 8));
+    }
+#pragma unroll
+    for (int h = 0; h < 8; ++h) c[h] = n[h];
+  }
+}
+
 // Hillis-Steele inclusive scan of one 128-position tile (p = h * 64 + lane).
 template <typename T>
 __device__ __forceinline__ void hs_scan128(T c[2], int l) {
