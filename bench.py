@@ -137,7 +137,7 @@ TRAFFIC_KERNELS = {
     "sort_c2": ("tx::radix_sort_rows_kernel", "tx::gather_row_lds_kernel"),
     "prefill_c5": ("tx::softmax_topk_kernel",),
     "sort_wide": ("tx::sort_chunks_kernel", "tx::bucket_", "tx::merge_runs_kernel"),
-    "topk_router": ("tx::topk_short_block_kernel",),
+    "topk_router": ("tx::topk_lanes_kernel",),
     "cumsum_long": ("tx::cumsum_",),
 }
 EXTRA_CONFIGS = ("topk_c3", "prefill_c5", "sort_c2")
@@ -507,7 +507,7 @@ def _topk_router(torch, np, _lib, dev, s_handle, gen, nbuf):
     w.rows, w.dtype, w.shape = rows, "f32", (rows, cols)
     w.alg_bytes = rows * cols * 4 + rows * k * 8  # logits in, values and indices out
     w.workload = "exact top-k (tax.top_k) k=8: f32 [65536,128] ~ N(0,1) (router-sized rows)"
-    w.kernel = "topk_short_block_kernel<0, 128, 2>"
+    w.kernel = "topk_lanes_kernel<0, 8, 8, 16>"
     w.cpu_batch = 4096
 
     def launch(i):

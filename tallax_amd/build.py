@@ -26,6 +26,7 @@ LIB_PATH = OUT_DIR / LIB_NAME
 SOURCES = [
     "capi.hip",
     "row_select.hip",
+    "topk_short.hip",
     "scan_gather.hip",
     "sort_rows.hip",
     "sort_wide.hip",

@@ -1958,146 +1958,6 @@ int launch_segment_lists(const void* x, int dt, int64_t rows, int64_t cols, int 
   return launch_status("segment lists");
 }
 
-// ---------------------------------------------------------------------------
-// Short rows (at most 2048 elements): every row sorted whole.  A 1024-thread
-// select workgroup per row spends its fixed latency on a few hundred
-// elements (f32, k = 8: [65536, 128] 1444 us, [65536, 512] 1703 us,
-// [32768, 1024] 1051 us that way).  Records order the output ascending:
-// (~select key) << 32 | column, the select key ordering values as the
-// reference's strict `>` admits them (top_k.py:64: -0 == +0, NaN below -inf),
-// ties by lowest column; padding records (all ones) go last.  Values at or
-// below finfo(dtype).min, and NaNs, come out as finfo.min.
-//   * rows of at most 32: one thread per row, a register bitonic network;
-//   * longer rows: block_bitonic_sort_c over P = 64 .. 2048 slots, E records
-//     per thread (one wave up to P = 512, then 128 and 256 threads).
-// ---------------------------------------------------------------------------
-constexpr int kTopkShortCols = 2048;
-
-// Whole-row sorts pay off at any row count up to 256 elements; beyond that
-// only with many rows, where the select kernel's per-row latency adds up
-// (f32, k = 8, select -> sort: [65536, 512] 1711 -> 182 us, [32768, 1024]
-// 1056 -> 223, [16384, 2048] 332 -> 271, [4096, 2048] 81 -> 80; few rows
-// lose: [64, 1024] 10.3 -> 12.0, [256, 2048] 6.7 -> 14.8, [1024, 2048]
-// k = 64 20.9 -> 28.9).
-static bool topk_short_route(int64_t rows, int64_t cols) {
-  return cols <= 256 || (cols <= 1024 && rows >= 512) || (cols <= kTopkShortCols && rows >= 8192);
-}
-
-__device__ __forceinline__ uint32_t topk_select_key(uint32_t b) {  // b: float32 bits
-  const uint32_t a = b & 0x7FFFFFFFu;
-  if (a > 0x7F800000u) return 1u;
-  if (a == 0u) return 0x80000000u;
-  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t topk_f32_bits(const void* x, int64_t i) {
-  return DT == kBF16 ? (uint32_t)((const uint16_t*)x)[i] << 16 : ((const uint32_t*)x)[i];
-}
-
-// Output position i of a row: positions >= k_rows[row] (when k_rows is
-// given) keep the index and take the replacement value (float32 bits).
-struct TopkShortOut {
-  void* vals;
-  int32_t* idx;
-  const int32_t* k_rows;
-  uint32_t replace_bits;
-};
-
-template <int DT>
-__device__ __forceinline__ void topk_short_out(uint64_t rec, const void* x, int64_t base, int64_t row, int i, int k,
-                                               const TopkShortOut& ot) {
-  const int64_t o = row * k + i;
-  void* out_vals = ot.vals;
-  int32_t* out_idx = ot.idx;
-  const uint32_t col = (uint32_t)rec;
-  uint32_t b = topk_f32_bits<DT>(x, base + col);
-  const uint32_t kmin = topk_select_key(DT == kBF16 ? 0xFF7F0000u : 0xFF7FFFFFu);
-  if (topk_select_key(b) <= kmin) b = DT == kBF16 ? 0xFF7F0000u : 0xFF7FFFFFu;
-  if (ot.k_rows && i >= ot.k_rows[row]) b = ot.replace_bits;
-  out_idx[o] = (int32_t)col;
-  if (DT == kBF16) ((uint16_t*)out_vals)[o] = (uint16_t)(b >> 16);
-  else ((uint32_t*)out_vals)[o] = b;
-}
-
-template <int DT, int NC>
-__global__ __launch_bounds__(256) void topk_short_thread_kernel(const void* __restrict__ x, int64_t rows, int cols,
-                                                                int k, TopkShortOut ot) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= rows) return;
-  const int64_t base = row * cols;
-  uint64_t v[NC];
-#pragma unroll
-  for (int i = 0; i < NC; ++i)
-    v[i] = i < cols ? ((uint64_t)~topk_select_key(topk_f32_bits<DT>(x, base + i)) << 32) | (uint32_t)i : ~0ull;
-#pragma unroll
-  for (int kk = 2; kk <= NC; kk <<= 1) {
-#pragma unroll
-    for (int j = kk >> 1; j > 0; j >>= 1) {
-#pragma unroll
-      for (int i = 0; i < NC; ++i) {
-        const int o = i ^ j;
-        if (o > i) {
-          const uint64_t a = v[i], b = v[o];
-          const bool sw = (i & kk) == 0 ? a > b : a < b;
-          v[i] = sw ? b : a;
-          v[o] = sw ? a : b;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < NC; ++i)
-    if (i < k) topk_short_out<DT>(v[i], x, base, row, i, k, ot);
-}
-
-template <int DT, int P, int E>
-__global__ __launch_bounds__(P / E) void topk_short_block_kernel(const void* __restrict__ x, int cols, int k,
-                                                                 TopkShortOut ot) {
-  __shared__ uint64_t lds[P];
-  const int64_t row = blockIdx.x;
-  const int64_t base = row * cols;
-  const int t = threadIdx.x;
-  uint64_t v[E];
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const int i = t * E + r;
-    v[r] = i < cols ? ((uint64_t)~topk_select_key(topk_f32_bits<DT>(x, base + i)) << 32) | (uint32_t)i : ~0ull;
-  }
-  block_bitonic_sort_c<uint64_t, E, P, false>(v, lds);
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const int i = t * E + r;
-    if (i < k) topk_short_out<DT>(v[r], x, base, row, i, k, ot);
-  }
-}
-
-template <int DT>
-static int launch_topk_short(const void* x, int64_t rows, int64_t cols, int k, const TopkShortOut& ot,
-                             hipStream_t s) {
-  const int c = (int)cols;
-  if (cols <= 32) {
-    const unsigned grid = (unsigned)((rows + 255) / 256);
-    if (cols <= 16)
-      hipLaunchKernelGGL((topk_short_thread_kernel<DT, 16>), dim3(grid), dim3(256), 0, s, x, rows, c, k, ot);
-    else
-      hipLaunchKernelGGL((topk_short_thread_kernel<DT, 32>), dim3(grid), dim3(256), 0, s, x, rows, c, k, ot);
-  } else if (cols <= 64) {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 64, 1>), dim3((unsigned)rows), dim3(64), 0, s, x, c, k, ot);
-  } else if (cols <= 128) {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 128, 2>), dim3((unsigned)rows), dim3(64), 0, s, x, c, k, ot);
-  } else if (cols <= 256) {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 256, 4>), dim3((unsigned)rows), dim3(64), 0, s, x, c, k, ot);
-  } else if (cols <= 512) {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 512, 8>), dim3((unsigned)rows), dim3(64), 0, s, x, c, k, ot);
-  } else if (cols <= 1024) {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 1024, 8>), dim3((unsigned)rows), dim3(128), 0, s, x, c, k, ot);
-  } else {
-    hipLaunchKernelGGL((topk_short_block_kernel<DT, 2048, 8>), dim3((unsigned)rows), dim3(256), 0, s, x, c, k, ot);
-  }
-  return launch_status("top-k (short rows)");
-}
-
 static int check_common(const void* x, int dt, int64_t rows, int64_t cols) {
   if (!x) { set_error("null input pointer"); return kInvalidArgument; }
   if (dt != kF32 && dt != kBF16) { set_error("dtype %d not supported (f32=0, bf16=1)", dt); return kUnsupported; }
@@ -2186,10 +2046,9 @@ int tallax_topk(const void* x, int dtype, int64_t rows, int64_t cols, int64_t k,
   if (rows == 0) return kOk;
   if (dtype == kI32)
     return topk_i32(x, rows, cols, k, nullptr, 0.0, out_vals, out_idx, workspace, workspace_bytes, stream, "tallax_topk");
-  if (topk_short_route(rows, cols)) {
+  if (topk_short_route(rows, cols, (int)k)) {
     const TopkShortOut ot = {out_vals, out_idx, nullptr, 0u};
-    return dtype == kF32 ? launch_topk_short<kF32>(x, rows, cols, (int)k, ot, stream)
-                         : launch_topk_short<kBF16>(x, rows, cols, (int)k, ot, stream);
+    return launch_topk_short(x, dtype, rows, cols, (int)k, ot, stream);
   }
   Plan p;
   st = plan_rows(rows, cols, dtype, &p);
@@ -2220,14 +2079,13 @@ int tallax_topk_replace(const void* x, int dtype, int64_t rows, int64_t cols, in
   if (dtype == kI32)
     return topk_i32(x, rows, cols, k, k_rows, replace_val, out_vals, out_idx, workspace, workspace_bytes, stream,
                     "tallax_topk_replace");
-  if (topk_short_route(rows, cols)) {
+  if (topk_short_route(rows, cols, (int)k)) {
     const float rf = (float)replace_val;
     uint32_t rb;
     const float rd = dtype == kBF16 ? round_to_bf16(rf) : rf;
     memcpy(&rb, &rd, sizeof(rb));
     const TopkShortOut ot = {out_vals, out_idx, k_rows, rb};
-    return dtype == kF32 ? launch_topk_short<kF32>(x, rows, cols, (int)k, ot, stream)
-                         : launch_topk_short<kBF16>(x, rows, cols, (int)k, ot, stream);
+    return launch_topk_short(x, dtype, rows, cols, (int)k, ot, stream);
   }
   Plan p;
   st = plan_rows(rows, cols, dtype, &p);

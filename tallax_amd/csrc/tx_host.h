@@ -57,6 +57,19 @@ int segment_lists_plan(int64_t rows, int64_t cols, int dt, int min_seg, int* nse
 int launch_segment_lists(const void* x, int dt, int64_t rows, int64_t cols, int nseg, int maxv, int64_t vps,
                          uint64_t* lists, hipStream_t s);
 
+// Output position i of a short-row top-k (topk_short.hip): positions >=
+// k_rows[row] (when k_rows is given) keep the index and take the replacement
+// value (float32 bits).
+struct TopkShortOut {
+  void* vals;
+  int32_t* idx;
+  const int32_t* k_rows;
+  uint32_t replace_bits;
+};
+bool topk_short_route(int64_t rows, int64_t cols, int k);
+int launch_topk_short(const void* x, int dt, int64_t rows, int64_t cols, int k, const TopkShortOut& ot,
+                      hipStream_t s);
+
 // Arguments of a row sort (sort_rows.hip, sort_wide.hip).
 struct SortArgs {
   const void* key;
