@@ -80,8 +80,7 @@ struct SelArgs {
   uint64_t* ws_lists;
   int lists_only;  // write the segment list even when a row is one segment
   int64_t col_offset;   // added to every column index of a written list (a vocabulary shard's first column)
-  int64_t part_cols;    // whole-row kernel on row parts: part p of a row holds columns [p * part_cols, (p + 1) * part_cols)
-  int nparts;
+  int part_cols;        // whole-row kernel: part p of a row holds columns [p * part_cols, (p + 1) * part_cols)
   int list_k;           // whole-row kernel: places of the row's (or part's) list that are read (64; 0: all 128)
   uint64_t* out_lists;  // merge kernel, lists_only: the merged list of each row, [rows][128]
   // sampler
@@ -1349,9 +1348,9 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
   const int64_t row = blockIdx.x;
   // row parts (SAMPLE = false only): workgroup (row, part) of a two-dimensional
-  // grid; the row's last part may be shorter
-  const int64_t c0 = !SAMPLE && a.nparts > 1 ? (int64_t)blockIdx.y * a.part_cols : 0;
-  const int cols = (int)(!SAMPLE && a.nparts > 1 ? (a.cols - c0 < a.part_cols ? a.cols - c0 : a.part_cols) : a.cols);
+  // grid; the row's last part may be shorter (part_cols = cols: whole rows)
+  const int64_t c0 = SAMPLE ? 0 : (int64_t)((uint64_t)blockIdx.y * (uint32_t)a.part_cols);
+  const int left = (int)(a.cols - c0), cols = SAMPLE || left < a.part_cols ? left : a.part_cols;
   const char* rowp = (const char*)a.x + (size_t)(row * a.cols + c0) * ES;
   const RowVec<ES> rv(rowp);
   const int nv = (cols + rv.mis + VEC - 1) / VEC;  // 1 <= nv <= kNTS * V (host plan)
@@ -1480,7 +1479,20 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   // reach it.  Their loads are issued first and arrive first, so L is posted
   // before waves 8..15 have their first vector, and those stage each vector
   // as it arrives.
+  // Rows too short for every lane of those waves to hold a vector share the
+  // places out by the vectors each wave holds; with equal quotas the empty
+  // waves' bound was 0, every element a candidate, and rows of more than 1024
+  // elements overflowed into the tie path (top-k k = 64: [256, 1500] f32
+  // 38.1 -> 7.0 us, [256, 2048] bf16 38.0 -> 6.3, [1024, 3000] bf16 146 -> 21).
+  // Rows of fewer vectors than places fit the candidate array whole.
   constexpr int NE = NW / 2;
+  int quota = kq / NE;  // kq is 64 or 128
+  bool bounds = true;   // this wave's bound counts
+  if (nv < NE * kWave) {  // block-uniform
+    const int nl = nv - w * kWave < kWave ? nv - w * kWave : kWave;
+    bounds = nl > 0;
+    quota = nv >= kq ? (kq * nl + nv - 1) / nv : kWave + 1;  // more than the wave's lanes: bound 0
+  }
   const bool early = w < NE;
   int32_t vmax[V];  // early waves: their vectors' maxima, kept for the staging
   {
@@ -1512,9 +1524,9 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
         }
       }
       uint32_t wl, wm;
-      wave_kth_and_max<KB>(tk, kq / NE, wl, wm);
+      wave_kth_and_max<KB>(tk, quota, wl, wm);
       if (l == 0) {
-        ss.wl[w] = wl;
+        ss.wl[w] = bounds ? wl : ~0u;
         ss.wm[w] = wm;
         __hip_atomic_fetch_or(&ss.posted, 1u << w, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
@@ -1836,20 +1848,20 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
   // parts: the whole-row kernel writes each part's list (no sampling), the
   // merge kernel finishes the row
   SelArgs h = a0;
+  h.part_cols = (int)a0.cols;
   // top-k with k <= 64 reads the first 64 places of a row's (or a part's) list
   if (!SAMPLE && !a0.lists_only && a0.k <= kWave) h.list_k = kWave;
   if (p.parts > 1) {
     h.nseg = 1;
     h.lists_only = 1;
-    h.part_cols = part_cols_of(a0.cols, p.parts, ElemT<DT>::VEC);
-    h.nparts = p.parts;
+    h.part_cols = (int)part_cols_of(a0.cols, p.parts, ElemT<DT>::VEC);
   }
   const SelArgs& a = h;
   if (p.nt == kNTS && p.parts > 1) {
     // every row and every part starts 16-byte aligned and fills its last vector
     // (the row's last part too: cols and part_cols both are whole vectors)
     const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0 ||
-                      (a.part_cols * ElemT<DT>::ES) % 16 != 0;
+                      ((int64_t)a.part_cols * ElemT<DT>::ES) % 16 != 0;
     const dim3 g((unsigned)a.rows, (unsigned)p.parts), b(kNTS);
     if (p.maxv == 19) {
       if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true>), g, b, 0, s, a);

@@ -61,3 +61,14 @@ def test_segments_with_few_eligible(gpu, rows, cols, k, dtype, kind):
 ])
 def test_uneven_parts(gpu, rows, cols, k, dtype, kind, parts):
     _check(gpu, rows, cols, k, dtype, kind, 1024, parts)
+
+
+# rows whose vectors do not fill the waves that give the bound: their shares of
+# the places at a few vectors per wave, a partial wave, and the last short row
+@pytest.mark.parametrize("cols,dtype", [(1025, "f32"), (1031, "f32"), (1300, "f32"), (2044, "f32"), (2049, "f32"),
+                                        (1025, "bf16"), (1100, "bf16"), (1528, "bf16"), (2050, "bf16"),
+                                        (4090, "bf16"), (4097, "bf16")])
+@pytest.mark.parametrize("k,kind", [(64, "normal"), (128, "normal"), (128, "masked_mix"), (100, "ints"),
+                                    (64, "sorted_desc"), (128, "special")])
+def test_bound_of_short_rows(gpu, cols, dtype, k, kind):
+    _check(gpu, 40, cols, k, dtype, kind, 1024, 1)
