@@ -13,8 +13,8 @@
 // the tie is the element's column (or 0x7FFFFFFF - column).  Records are
 // unique, so any correct sort of them gives exactly that order, and two
 // sorted runs merge without a stability rule.
-//   1. sort_chunks_kernel: one 512-thread workgroup sorts each 16384-record
-//      chunk of a row in LDS (a stable LSD radix sort on the key, 8-bit
+//   1. sort_chunks_kernel: one 512-thread workgroup sorts each 16384- or
+//      8192-record chunk of a row in LDS (a stable LSD radix sort on the key, 8-bit
 //      digits) and writes the sorted run to the workspace.
 //   2. merge_runs_kernel, ceil(log2(chunks)) passes: runs of length L are
 //      merged pairwise into runs of 2L, ping-ponging between two workspace
@@ -42,7 +42,6 @@ namespace tx {
 constexpr int kWideChunk = 16384;  // records per chunk sorted in LDS
 constexpr int kChunkNT = 512;
 constexpr int kChunkE = kWideChunk / kChunkNT;
-constexpr int kChunkLds = kWideChunk * 8 + 256 * (kChunkNT / kWave + 1) * 4;  // records + digit counters
 constexpr int kMergeNT = 256;
 constexpr int kMergeItems = 16;                      // outputs per thread
 constexpr int kMergeTile = kMergeNT * kMergeItems;   // outputs per workgroup
@@ -122,7 +121,7 @@ __device__ __forceinline__ void radix_sort_slots(uint64_t (&v)[E], uint64_t* buf
   }
 }
 
-// Pass 1: sorted runs of kWideChunk records, by a stable LSD radix sort on
+// Pass 1: sorted runs of CH = E * kChunkNT records, by a stable LSD radix sort on
 // the 32-bit key in 8-bit digits (radix_sort_slots: at most four passes; a
 // digit that every key of the chunk shares is skipped).  Slot p of the chunk
 // holds record (order bits << 32 | tie) of linear index p (column c0 + p, or
@@ -130,41 +129,42 @@ __device__ __forceinline__ void radix_sort_slots(uint64_t (&v)[E], uint64_t* buf
 // order of the full records; slots past the row hold all-ones records, which
 // stay last.  (Eight passes of 4-bit digits with per-thread packed counters
 // took 2.93 ms at [1024, 201088]; these four, 1.60 ms.)
-template <int DT, bool PERM>
+template <int DT, bool PERM, int E>
 __global__ __launch_bounds__(kChunkNT) void sort_chunks_kernel(SortArgs a, int nchunks, uint64_t* out) {
   constexpr int NW = kChunkNT / kWave;
+  constexpr int CH = E * kChunkNT;                     // records of a chunk
   extern __shared__ __align__(16) unsigned char smem[];
-  uint64_t* buf = (uint64_t*)smem;                     // kWideChunk records
-  uint32_t* hist = (uint32_t*)(buf + kWideChunk);      // 256 * HS counters
+  uint64_t* buf = (uint64_t*)smem;                     // CH records
+  uint32_t* hist = (uint32_t*)(buf + CH);      // 256 * HS counters
   __shared__ uint32_t wsum[NW];
   __shared__ uint32_t red[2][NW];
   const int t = threadIdx.x, l = lane_id(), w = t / kWave;
   const int64_t row = blockIdx.x / (unsigned)nchunks;
   const int c = (int)(blockIdx.x - row * nchunks);
   const int64_t base = row * a.cols;
-  const int64_t c0 = (int64_t)c * kWideChunk;
-  const int n = (int)min((int64_t)kWideChunk, a.cols - c0);
+  const int64_t c0 = (int64_t)c * CH;
+  const int n = (int)min((int64_t)CH, a.cols - c0);
   // records in slot order (coalesced reads, every load of the chunk in
   // flight at once), and which key bits vary
   uint32_t kand = ~0u, kor = 0u;
-  uint64_t v[kChunkE];
+  uint64_t v[E];
   {
-    uint32_t raw[kChunkE];
-    int32_t src[kChunkE];
+    uint32_t raw[E];
+    int32_t src[E];
 #pragma unroll
-    for (int r = 0; r < kChunkE; ++r) {
-      const int L = w * (kChunkE * kWave) + r * kWave + l;
+    for (int r = 0; r < E; ++r) {
+      const int L = w * (E * kWave) + r * kWave + l;
       src[r] = (int32_t)(c0 + (a.ties_desc ? n - 1 - L : L));
       if (PERM && L < n) src[r] = a.perm_in[base + src[r]];
     }
 #pragma unroll
-    for (int r = 0; r < kChunkE; ++r) {
-      const int L = w * (kChunkE * kWave) + r * kWave + l;
+    for (int r = 0; r < E; ++r) {
+      const int L = w * (E * kWave) + r * kWave + l;
       raw[r] = L < n ? key_bits_at<DT>(a.key, base + src[r]) : 0u;
     }
 #pragma unroll
-    for (int r = 0; r < kChunkE; ++r) {
-      const int L = w * (kChunkE * kWave) + r * kWave + l;
+    for (int r = 0; r < E; ++r) {
+      const int L = w * (E * kWave) + r * kWave + l;
       v[r] = ~0ull;
       if (L < n) {
         uint32_t k = order_from_bits(raw[r], DT);
@@ -192,11 +192,11 @@ __global__ __launch_bounds__(kChunkNT) void sort_chunks_kernel(SortArgs a, int n
   // bfloat16 keys: the low 16 order bits follow from the high 16 (as in
   // sort_row_radix_kernel), so only the high digits are sorted
   const uint32_t varying = (kand ^ kor) & (DT == kBF16 ? 0xFFFF0000u : ~0u);
-  radix_sort_slots<kChunkE, kChunkNT>(v, buf, hist, wsum, varying, n);
+  radix_sort_slots<E, kChunkNT>(v, buf, hist, wsum, varying, n);
   uint64_t* dst = out + base + c0;
 #pragma unroll
-  for (int r = 0; r < kChunkE; ++r) {
-    const int L = w * (kChunkE * kWave) + r * kWave + l;
+  for (int r = 0; r < E; ++r) {
+    const int L = w * (E * kWave) + r * kWave + l;
     if (L < n) dst[L] = v[r];
   }
 }
@@ -363,9 +363,8 @@ __global__ __launch_bounds__(kMergeNT) void merge_runs_kernel(SortArgs a, const 
 // ---------------------------------------------------------------------------
 // Multiway merge by splitters (rows of 3 to kBucketMaxRuns chunks): one pass
 // instead of ceil(log2 chunks) pairwise merge passes.
-//   * bucket_split_kernel, one workgroup per row: every kBucketStride-th record
-//     of every sorted run is a sample (record (a + 1) G - 1 of a run, G the
-//     stride); the samples (at most 4096) are sorted by a block bitonic
+//   * bucket_split_kernel, one workgroup per row: every G-th record of every
+//     sorted run is a sample (record (a + 1) G - 1 of a run); the samples (at most 4096) are sorted by a block bitonic
 //     network, and every m-th one of them in that order is a splitter s_k.
 //     For every splitter and run, the run's first position p_kj with a record
 //     >= s_k: the run's samples below s_k, c, put it in [c G, (c + 1) G), so a
@@ -375,36 +374,40 @@ __global__ __launch_bounds__(kMergeNT) void merge_runs_kernel(SortArgs a, const 
 //     bucket never exceeds (m + runs) G records: m is chosen so that this is
 //     the bucket kernel's capacity.  The table holds every p_kj and each
 //     bucket's first output rank, sum_j p_kj.
+//     G is 64 where the samples fit: the finer they are, the fuller the buckets
+//     (79 % of the capacity at 13 runs against 58 % with G = 256).  Few rows take
+//     smaller buckets, so that they fill the chip.
 //   * bucket_sort_kernel, one workgroup per (row, bucket): the bucket's part of
-//     every run is loaded, run after run in tie order (chunk j holds columns
-//     [j, j + 1) kWideChunk: ascending ties take the runs in order, descending
-//     ones in reverse).  Inside one run the records are sorted, and between
-//     runs records of equal keys then come in tie order.  So the stable radix sort by the key
-//     alone (radix_sort_slots) gives the records' order, and the outputs
-//     (permutation, keys, gathered second key) are written at the bucket's
-//     first output rank.
+//     every run, in tie order, sorted in LDS; the outputs (permutation, keys,
+//     gathered second key) are written from the bucket's first output rank.
 // Traffic: the chunk pass (4 bytes in, 8 out per element), then 8 in and the
 // outputs out: 28 bytes per element with keys and indices out, against 76 for
-// four pairwise merge passes at [1024, 201088].
+// four pairwise merge passes at [1024, 201088].  There the three kernels take
+// 1000 + 272 + 1197 us: chunks bound by LDS (bank conflicts of the scattered
+// records), buckets by the latency of their loads and LDS steps.
 // ---------------------------------------------------------------------------
-constexpr int kBucketStride = 256;       // G: records between samples
+constexpr int kBucketStride = 256;       // G: records between samples ...
+constexpr int kBucketStrideFine = 64;    // ... of rows of at most kSplitSamples * 64 elements
 constexpr int kBucketMaxRuns = 56;       // (m >= 8) + runs <= 64: buckets of at most 64 G = 16384 records
 constexpr int kSplitNT = 1024;
 constexpr int kSplitSamples = 4096;      // >= kBucketMaxRuns * kWideChunk / kBucketStride
-constexpr int kBucketNT = 512;
+constexpr int kBucketPad = 4;            // records read at a time in a bin
+constexpr uint32_t kBinMost = 24;        // records in one bin past which the radix sort takes over
 static_assert(kBucketMaxRuns * (kWideChunk / kBucketStride) <= kSplitSamples, "every sample fits the sort");
 
 struct BucketPlan {
   int runs;     // chunks of a row
+  int chunk;    // records of a run (the row's last one may be shorter)
+  int G;        // records between samples of a run
   int samples;  // S: samples of a row
   int m;        // samples per bucket
   int K;        // buckets of a row
-  int E;        // records per thread of the bucket kernel (capacity E * kBucketNT)
+  int cap;      // records a bucket may hold: 4096, 8192 or 16384
 };
 
-__host__ __device__ inline int run_len(int64_t cols, int j) {
-  const int64_t left = cols - (int64_t)j * kWideChunk;
-  return (int)(left < kWideChunk ? left : kWideChunk);
+__host__ __device__ inline int run_len(int64_t cols, int chunk, int j) {
+  const int64_t left = cols - (int64_t)j * chunk;
+  return (int)(left < chunk ? left : chunk);
 }
 
 __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
@@ -416,15 +419,8 @@ __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, Buck
   const int t = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int64_t base = row * a.cols;
-  const int R = bp.runs, G = kBucketStride;
-  if (t == 0) {
-    int acc = 0;
-    for (int j = 0; j < R; ++j) {
-      sp[j] = acc;
-      acc += run_len(a.cols, j) / G;
-    }
-    sp[R] = acc;
-  }
+  const int R = bp.runs, G = bp.G;
+  if (t <= R) sp[t] = t < R ? t * (bp.chunk / G) : bp.samples;
   for (int k = t; k <= bp.K; k += kSplitNT) soff[k] = 0;
   __syncthreads();
   // sample i = 4t + r: run j with sp[j] <= i < sp[j + 1], record (i - sp[j] + 1) G - 1 of it
@@ -434,9 +430,8 @@ __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, Buck
     const int i = 4 * t + r;
     v[r] = ~0ull;
     if (i < bp.samples) {
-      int j = 0;
-      while (sp[j + 1] <= i) ++j;
-      v[r] = runs[base + (int64_t)j * kWideChunk + (int64_t)(i - sp[j] + 1) * G - 1];
+      const int j = i / (bp.chunk / G);  // every run but the last has chunk / G samples
+      v[r] = runs[base + (int64_t)j * bp.chunk + (int64_t)(i - sp[j] + 1) * G - 1];
       per[i] = v[r];
     }
   }
@@ -448,7 +443,7 @@ __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, Buck
   int32_t* tp = table + row * (int64_t)(bp.K + 1) * (R + 1);  // [(K + 1) R] positions, then [K + 1] offsets
   for (int q = t; q < (bp.K + 1) * R; q += kSplitNT) {
     const int k = q / R, j = q - k * R;
-    const int len = run_len(a.cols, j);
+    const int len = run_len(a.cols, bp.chunk, j);
     int pos;
     if (k == 0) {
       pos = 0;
@@ -466,7 +461,7 @@ __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, Buck
       const int c = lo - sp[j];
       // first record >= sk in [c G, min((c + 1) G - 1, len)]
       int l0 = c * G, h0 = c < sp[j + 1] - sp[j] ? (c + 1) * G - 1 : len;
-      const uint64_t* rj = runs + base + (int64_t)j * kWideChunk;
+      const uint64_t* rj = runs + base + (int64_t)j * bp.chunk;
       while (l0 < h0) {
         const int mid = (l0 + h0) >> 1;
         if (rj[mid] < sk) l0 = mid + 1;
@@ -481,17 +476,47 @@ __global__ __launch_bounds__(kSplitNT) void bucket_split_kernel(SortArgs a, Buck
   for (int k = t; k <= bp.K; k += kSplitNT) tp[(bp.K + 1) * R + k] = soff[k];
 }
 
-template <int E>
-__global__ __launch_bounds__(kBucketNT) void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
+// Bins of a bucket of E * NT records: half as many, which fit the radix sort's
+// counters (16-bit, and the end of the last one).  Larger buckets (E = 32, rows
+// of more than 24 runs) take the radix sort: the bins' registers would spill.
+constexpr int bucket_bins(int nt, int e) { return e <= 16 ? 8 * nt : 0; }
+static_assert(bucket_bins(256, 16) * 2 + 4 <= 256 * 5 * 4 && bucket_bins(512, 16) * 2 + 4 <= 256 * 9 * 4, "bins fit");
+
+// Multiplier that spreads key offsets 0 .. range over the bins: offset * scale >> 32
+// is below BINS and ascends with the offset.
+template <int BINS>
+__device__ __forceinline__ uint32_t bin_scale(uint32_t range) {
+  if (range < (uint32_t)BINS) return ~0u;
+  return (uint32_t)(((uint64_t)BINS << 32) / ((uint64_t)range + 1u));
+}
+
+// One workgroup per (row, bucket).  Slot L of the bucket is record L - s_off[i] of
+// its part of the i-th run in tie order: chunk j holds columns [j, j + 1) * chunk,
+// so with descending ties (tie = kTieMask - column) the last run comes first.
+//
+// A bucket's keys lie in a narrow range of the row's, so they spread nearly
+// evenly over bins of equal key ranges: one atomic per record gives it a place
+// in its bin, a scan the bins' starts, and after one move through LDS a
+// record's rank is its bin's start + the smaller records of its bin.  That is
+// one pass and five barriers, against three to four radix passes of five
+// ([1024, 201088] f32, buckets of 8192: 1792 -> 1210 us; of 4096, four
+// workgroups to a CU: 994).
+// bf16 keys, key ranges of few values and bunched keys pile up in the bins and
+// take the stable radix sort on the key.
+template <int NT, int E, int DT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(E <= 16 ? 4 : 2, 8)))
+void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
                                                                 const int32_t* table) {
-  constexpr int NW = kBucketNT / kWave;
-  constexpr int CAP = E * kBucketNT;
+  constexpr int NW = NT / kWave;
+  constexpr int BINS = bucket_bins(NT, E);  // 0: the radix sort only
+  constexpr int CAP = E * NT;
   extern __shared__ __align__(16) unsigned char smem[];
-  uint64_t* buf = (uint64_t*)smem;                 // CAP records
-  uint32_t* hist = (uint32_t*)(buf + CAP);         // 256 * (NW + 1) counters
+  uint64_t* buf = (uint64_t*)smem;                        // CAP records + kBucketPad
+  uint32_t* hist = (uint32_t*)(buf + CAP + kBucketPad);   // 256 * (NW + 1) counters, or the bins
   __shared__ uint32_t wsum[NW];
   __shared__ uint32_t red[2][NW];
-  __shared__ int s_lo[kBucketMaxRuns], s_off[kBucketMaxRuns + 1];
+  __shared__ int s_off[kBucketMaxRuns + 1];
+  __shared__ uint32_t s_src[kBucketMaxRuns];  // slot L of run i is the row's record s_src[i] + L
   const int t = threadIdx.x, l = lane_id(), w = t / kWave;
   const int R = bp.runs;
   const int64_t row = blockIdx.x / (unsigned)bp.K;
@@ -499,107 +524,211 @@ __global__ __launch_bounds__(kBucketNT) void bucket_sort_kernel(SortArgs a, Buck
   const int64_t base = row * a.cols;
   const int32_t* tp = table + row * (int64_t)(bp.K + 1) * (R + 1);
   if (w == 0) {  // the bucket's range in each run and its slots, by a wave scan
-    // runs in tie order: chunk j holds columns [j, j + 1) * kWideChunk, so
-    // with descending ties (tie = kTieMask - column) the last run comes first
+    const int j = a.ties_desc ? R - 1 - l : l;
     int lo = 0, sz = 0;
     if (l < R) {
-      const int j = a.ties_desc ? R - 1 - l : l;
       lo = tp[k * R + j];
       sz = tp[(k + 1) * R + j] - lo;
     }
     int tot;
     const int pre = wave_exscan_i32(sz, tot);
     if (l < R) {
-      s_lo[l] = lo;
       s_off[l] = pre;
+      s_src[l] = (uint32_t)(j * bp.chunk + lo - pre);
     }
     if (l == 0) s_off[R] = tot;
   }
+  uint32_t* bins = hist;  // BINS 16-bit counters, two to a word
+  if (DT != kBF16)
+    for (int q = t; q < BINS / 2; q += NT) bins[q] = 0u;
   __syncthreads();
   const int n = s_off[R];  // at most CAP (the split's bound)
   if (n > CAP) return;     // never taken; keeps a broken table from writing past the LDS buffer
   const int64_t o0 = tp[(bp.K + 1) * R + k];
-  // slot L is record L - s_off[i] of the bucket's part of the i-th run (in tie
-  // order); the slots of a thread ascend, so its run index only moves up
-  uint32_t kand = ~0u, kor = 0u;
+  uint32_t kmin = ~0u, kmax = 0u;
   uint64_t v[E];
   {
-    const uint64_t* src[E];
+    // a row's records span less than 2^32 bytes: 32-bit offsets from its start
+    const char* rr = (const char*)(runs + base);
     int i = 0;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const int L = w * (E * kWave) + r * kWave + l;
-      src[r] = nullptr;
+      const int L = r * NT + t;
+      v[r] = ~0ull;
       if (L < n) {
-        while (s_off[i + 1] <= L) ++i;
-        const int j = a.ties_desc ? R - 1 - i : i;
-        src[r] = runs + base + (int64_t)j * kWideChunk + s_lo[i] + (L - s_off[i]);
+        while (s_off[i + 1] <= L) ++i;  // a thread's slots ascend
+        v[r] = *(const uint64_t*)(rr + (s_src[i] + (uint32_t)L) * 8u);
       }
     }
 #pragma unroll
-    for (int r = 0; r < E; ++r) v[r] = src[r] ? *src[r] : ~0ull;
-#pragma unroll
     for (int r = 0; r < E; ++r) {
-      if (src[r]) {
-        kand &= (uint32_t)(v[r] >> 32);
-        kor |= (uint32_t)(v[r] >> 32);
+      if (r * NT + t < n) {
+        const uint32_t key = (uint32_t)(v[r] >> 32);
+        kmin = key < kmin ? key : kmin;
+        kmax = key > kmax ? key : kmax;
       }
     }
   }
-  kand = wave_and_u32(kand);
-  kor = wave_or_u32(kor);
+  kmin = wave_min_u32(kmin);
+  kmax = wave_max_u32(kmax);
   if (l == 0) {
-    red[0][w] = kand;
-    red[1][w] = kor;
+    red[0][w] = kmin;
+    red[1][w] = kmax;
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    kand &= red[0][i];
-    kor |= red[1][i];
+    kmin = red[0][i] < kmin ? red[0][i] : kmin;
+    kmax = red[1][i] > kmax ? red[1][i] : kmax;
   }
-  radix_sort_slots<E, kBucketNT>(v, buf, hist, wsum, (kand ^ kor) & (a.key_dtype == kBF16 ? 0xFFFF0000u : ~0u), n);
-  // outputs at ranks o0 + slot: the source column, then the sorted key and
-  // the gathered second key, each batch of dependent loads in flight at once
-  int32_t col[E];
+  kmin = __builtin_amdgcn_readfirstlane(kmin);
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+  const uint32_t scale = bin_scale<BINS>(kmax - kmin);
+  auto bin_of = [&](uint64_t x) -> uint32_t { return __umulhi((uint32_t)(x >> 32) - kmin, scale); };
+  uint32_t bin_most = ~0u;
+  uint32_t pb[E];  // place in the bin << 16 | bin
+  if constexpr (DT != kBF16 && BINS > 0) {
+  if (kmax - kmin >= (uint32_t)n / 4u) {  // block-uniform
 #pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const int L = w * (E * kWave) + r * kWave + l;
-    col[r] = 0;
-    if (L < n) {
-      const uint32_t tie = (uint32_t)v[r];
-      const int32_t pos = (int32_t)(a.ties_desc ? kTieMask - tie : tie);
-      col[r] = a.perm_in ? a.perm_in[base + pos] : pos;
+    for (int r = 0; r < E; ++r) {
+      pb[r] = 0u;
+      if (r * NT + t < n) {
+        const uint32_t b = bin_of(v[r]), sh = (b & 1u) * 16u;
+        pb[r] = ((atomicAdd(&bins[b >> 1], 1u << sh) >> sh) << 16) | b;
+      }
+    }
+    __syncthreads();
+    constexpr int PW = BINS / 2 / NT;  // words per thread
+    uint32_t cw[PW], most = 0u;
+    int sum = 0;
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+      cw[q] = bins[t * PW + q];
+      const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
+      sum += (int)(lo + hi);
+      most = max(most, max(lo, hi));
+    }
+    int tot;
+    const int pre = wave_exscan_i32(sum, tot);
+    most = wave_max_u32(most);
+    if (l == 0) {
+      wsum[w] = (uint32_t)tot;
+      red[0][w] = most;
+    }
+    __syncthreads();
+    uint32_t run = (uint32_t)pre;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      run += i < w ? wsum[i] : 0u;
+      most = max(most, red[0][i]);
+    }
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+      const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
+      bins[t * PW + q] = run | ((run + lo) << 16);  // the bins' starts, below 2^16
+      run += lo + hi;
+    }
+    if (t == 0) bins[BINS / 2] = (uint32_t)n;  // the end of the last bin
+    bin_most = __builtin_amdgcn_readfirstlane(most);
+  }
+  }
+  const bool spread = bin_most <= kBinMost;  // block-uniform
+  const uint16_t* start = (const uint16_t*)bins;
+  __syncthreads();
+  if (spread) {
+#pragma unroll
+    for (int r = 0; r < E; ++r)
+      if (r * NT + t < n) buf[start[pb[r] & 0xFFFFu] + (pb[r] >> 16)] = v[r];
+    if (t < kBucketPad) buf[n + t] = ~0ull;  // read past the last bin: larger than any record
+  } else {
+    // the slots in the radix sort's order, then back
+#pragma unroll
+    for (int r = 0; r < E; ++r)
+      if (r * NT + t < n) buf[r * NT + t] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      const int L = w * (E * kWave) + r * kWave + l;
+      v[r] = L < n ? buf[L] : ~0ull;
+    }
+    __syncthreads();  // the radix sort clears its counters over the bins and moves over buf
+    uint32_t varying = kmin == kmax ? 0u : 0xFFFFFFFFu >> __clz((int)(kmin ^ kmax));
+    if (DT == kBF16) varying &= 0xFFFF0000u;  // the low order bits of a bf16 key follow from the high
+    radix_sort_slots<E, NT>(v, buf, hist, wsum, varying, n);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      const int L = w * (E * kWave) + r * kWave + l;
+      if (L < n) buf[L] = v[r];
     }
   }
+  __syncthreads();
+  // outputs at o0 + rank: the source column, the sorted key and the gathered
+  // second key (32-bit offsets from the bucket's first output)
+  const int64_t ob = base + o0;
+  int32_t* po = a.perm_out + ob;
+  const uint32_t tmask = a.ties_desc ? kTieMask : 0u, dmask = a.descending ? ~0u : 0u;
+  char* ko = (char*)a.key_out + ob * (DT == kBF16 && a.key_out_dtype == kBF16 ? 2 : 4);
+  auto rank_of = [&](uint64_t x, int L) -> uint32_t {
+    if (!spread) return (uint32_t)L;
+    const uint32_t b = bin_of(x);
+    uint32_t k0 = start[b];
+    const uint32_t s1 = start[b + 1];
+    // records past the bin's end are larger: only the loop's end needs it
+    for (uint32_t i = k0; i < s1; i += kBucketPad) {
+      uint64_t m[kBucketPad];
+#pragma unroll
+      for (int u = 0; u < kBucketPad; ++u) m[u] = buf[i + u];
+#pragma unroll
+      for (int u = 0; u < kBucketPad; ++u) k0 += m[u] < x ? 1u : 0u;
+    }
+    return k0;
+  };
+  if (!a.perm_in && !a.aux_out) {
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      const int L = r * NT + t;
+      if (L >= n) continue;
+      const uint64_t x = buf[L];
+      const uint32_t k0 = rank_of(x, L);
+      po[k0] = (int32_t)((uint32_t)x ^ tmask);
+      if (a.key_out) store_sorted(ko, a.key_out_dtype, DT, k0, (uint32_t)(x >> 32) ^ dmask);
+    }
+    return;
+  }
+  // composed with an incoming permutation, or a second key to gather: each
+  // batch of dependent loads in flight at once
+  uint32_t rank[E], col[E];
 #pragma unroll
   for (int r = 0; r < E; ++r) {
-    const int L = w * (E * kWave) + r * kWave + l;
+    const int L = r * NT + t;
+    rank[r] = 0u;
+    col[r] = 0u;
     if (L >= n) continue;
-    a.perm_out[base + o0 + L] = col[r];
-    if (a.key_out) {
-      uint32_t key = (uint32_t)(v[r] >> 32);
-      if (a.descending) key = ~key;
-      store_sorted(a.key_out, a.key_out_dtype, a.key_dtype, base + o0 + L, key);
-    }
+    const uint64_t x = buf[L];
+    rank[r] = rank_of(x, L);
+    const uint32_t pos = (uint32_t)x ^ tmask;
+    col[r] = a.perm_in ? (uint32_t)a.perm_in[base + pos] : pos;
+    if (a.key_out) store_sorted(ko, a.key_out_dtype, DT, rank[r], (uint32_t)(x >> 32) ^ dmask);
   }
+#pragma unroll
+  for (int r = 0; r < E; ++r)
+    if (r * NT + t < n) po[rank[r]] = (int32_t)col[r];
   if (a.aux_out) {
     uint32_t u[E];
     if (a.aux_dtype == kBF16) {
 #pragma unroll
       for (int r = 0; r < E; ++r)
-        u[r] = w * (E * kWave) + r * kWave + l < n ? key_bits_at<kBF16>(a.aux, base + col[r]) : 0u;
+        u[r] = r * NT + t < n ? key_bits_at<kBF16>(a.aux, base + col[r]) : 0u;
     } else {
 #pragma unroll
       for (int r = 0; r < E; ++r)
-        u[r] = w * (E * kWave) + r * kWave + l < n ? key_bits_at<kF32>(a.aux, base + col[r]) : 0u;
+        u[r] = r * NT + t < n ? key_bits_at<kF32>(a.aux, base + col[r]) : 0u;
     }
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const int L = w * (E * kWave) + r * kWave + l;
-      if (L < n)
-        store_sorted(a.aux_out, a.aux_out_dtype, a.aux_dtype, base + o0 + L, order_from_bits(u[r], a.aux_dtype));
-    }
+    for (int r = 0; r < E; ++r)
+      if (r * NT + t < n)
+        store_sorted(a.aux_out, a.aux_out_dtype, a.aux_dtype, ob + rank[r], order_from_bits(u[r], a.aux_dtype));
   }
 }
 
@@ -730,16 +859,43 @@ static int launch_row_radix_dt(const SortArgs& a, int64_t rows, hipStream_t s) {
   return launch_row_radix_e<DT, PERM, 32>(a, rows, s);
 }
 
-template <int DT, bool PERM>
-static int launch_chunks(const SortArgs& a, int64_t rows, int64_t nchunks, uint64_t* out, hipStream_t s) {
-  const hipError_t attr = set_dynamic_lds_limit((const void*)sort_chunks_kernel<DT, PERM>, kChunkLds, s);
+template <int DT, bool PERM, int E>
+static int launch_chunks_one(const SortArgs& a, int64_t rows, int64_t nchunks, uint64_t* out, hipStream_t s) {
+  const int lds = E * kChunkNT * 8 + 256 * (kChunkNT / kWave + 1) * 4;  // records + digit counters
+  const hipError_t attr = set_dynamic_lds_limit((const void*)sort_chunks_kernel<DT, PERM, E>, lds, s);
   if (attr != hipSuccess) {
     set_error("hipFuncSetAttribute: %s", hipGetErrorString(attr));
     return kHipError;
   }
-  hipLaunchKernelGGL((sort_chunks_kernel<DT, PERM>), dim3((unsigned)(rows * nchunks)), dim3(kChunkNT), kChunkLds, s,
-                     a, (int)nchunks, out);
+  hipLaunchKernelGGL((sort_chunks_kernel<DT, PERM, E>), dim3((unsigned)(rows * nchunks)), dim3(kChunkNT), lds, s, a,
+                     (int)nchunks, out);
   return kOk;
+}
+template <int DT, bool PERM>
+static int launch_chunks(const SortArgs& a, int64_t rows, int64_t nchunks, int chunk, uint64_t* out, hipStream_t s) {
+  return chunk == kWideChunk ? launch_chunks_one<DT, PERM, kChunkE>(a, rows, nchunks, out, s)
+                             : launch_chunks_one<DT, PERM, kChunkE / 2>(a, rows, nchunks, out, s);
+}
+
+template <int NT, int E, int DT>
+static int launch_buckets_one(const SortArgs& a, int64_t rows, const BucketPlan& bp, const uint64_t* runs,
+                              const int32_t* table, hipStream_t s) {
+  const int lds = (E * NT + kBucketPad) * 8 + 256 * (NT / kWave + 1) * 4;
+  const hipError_t attr = set_dynamic_lds_limit((const void*)bucket_sort_kernel<NT, E, DT>, lds, s);
+  if (attr != hipSuccess) {
+    set_error("hipFuncSetAttribute: %s", hipGetErrorString(attr));
+    return kHipError;
+  }
+  hipLaunchKernelGGL((bucket_sort_kernel<NT, E, DT>), dim3((unsigned)(rows * bp.K)), dim3(NT), lds, s, a, bp, runs,
+                     table);
+  return kOk;
+}
+template <int DT>
+static int launch_buckets(const SortArgs& a, int64_t rows, const BucketPlan& bp, const uint64_t* runs,
+                          const int32_t* table, hipStream_t s) {
+  if (bp.cap == 4096) return launch_buckets_one<256, 16, DT>(a, rows, bp, runs, table, s);
+  if (bp.cap == 8192) return launch_buckets_one<512, 16, DT>(a, rows, bp, runs, table, s);
+  return launch_buckets_one<512, 32, DT>(a, rows, bp, runs, table, s);
 }
 
 static int wide_passes(int64_t cols) {
@@ -760,7 +916,15 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
     set_error("rows of %lld elements exceed the wide sort's limit of 2^31 - 1", (long long)cols);
     return kUnsupported;
   }
-  const int64_t nchunks = (cols + kWideChunk - 1) / kWideChunk;
+  // Rows whose samples fit at a stride of 64 take half chunks, two workgroups to a
+  // CU: one's LDS work covers the other's barriers (f32 [1024, 201088], chunks
+  // 1340 -> 1000 us; twice the runs cost the splitters 177 -> 272 and the buckets
+  // 994 -> 1197; in all 2510 -> 2405, [300, 50257] i32 282 -> 225, [14, 60833]
+  // 60 -> 55, bf16 [64, 131072] 140 -> 123).  Rows of two whole chunks stay on
+  // the merge pass: their workspace holds no splitter table.
+  const bool small = cols > 2 * kWideChunk && cols <= (int64_t)kSplitSamples * kBucketStrideFine;
+  const int chunk = small ? kWideChunk / 2 : kWideChunk;
+  const int64_t nchunks = (cols + chunk - 1) / chunk;
   const int64_t tiles = (cols + kMergeTile - 1) / kMergeTile;
   if (rows * tiles > 2147483647 || rows * nchunks > 2147483647) {
     set_error("sort of %lld x %lld elements needs more than 2^31 - 1 workgroups", (long long)rows, (long long)cols);
@@ -773,12 +937,12 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
     return kWorkspaceTooSmall;
   }
   uint64_t* buf[2] = {(uint64_t*)ws, (uint64_t*)ws + (size_t)rows * (size_t)cols};
-  int st = a.key_dtype == kBF16 ? (a.perm_in ? launch_chunks<kBF16, true>(a, rows, nchunks, buf[0], s)
-                                              : launch_chunks<kBF16, false>(a, rows, nchunks, buf[0], s))
-         : a.key_dtype == kI32  ? (a.perm_in ? launch_chunks<kI32, true>(a, rows, nchunks, buf[0], s)
-                                              : launch_chunks<kI32, false>(a, rows, nchunks, buf[0], s))
-                                : (a.perm_in ? launch_chunks<kF32, true>(a, rows, nchunks, buf[0], s)
-                                              : launch_chunks<kF32, false>(a, rows, nchunks, buf[0], s));
+  int st = a.key_dtype == kBF16 ? (a.perm_in ? launch_chunks<kBF16, true>(a, rows, nchunks, chunk, buf[0], s)
+                                              : launch_chunks<kBF16, false>(a, rows, nchunks, chunk, buf[0], s))
+         : a.key_dtype == kI32  ? (a.perm_in ? launch_chunks<kI32, true>(a, rows, nchunks, chunk, buf[0], s)
+                                              : launch_chunks<kI32, false>(a, rows, nchunks, chunk, buf[0], s))
+                                : (a.perm_in ? launch_chunks<kF32, true>(a, rows, nchunks, chunk, buf[0], s)
+                                              : launch_chunks<kF32, false>(a, rows, nchunks, chunk, buf[0], s));
   if (!st) st = launch_status("tallax_sort_rows (chunks)");
   if (st) return st;
   // rows of 3 .. kBucketMaxRuns chunks: the multiway merge by splitters
@@ -787,10 +951,19 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
   if (nchunks >= 3 && nchunks <= kBucketMaxRuns) {
     BucketPlan bp;
     bp.runs = (int)nchunks;
+    bp.chunk = chunk;
+    bp.G = small ? kBucketStrideFine : kBucketStride;
+    bp.cap = small ? 4096 : bp.runs <= 24 ? 8192 : 16384;
     bp.samples = 0;
-    for (int j = 0; j < bp.runs; ++j) bp.samples += run_len(cols, j) / kBucketStride;
-    bp.E = bp.runs <= 24 ? 16 : 32;                    // capacity 8192 or 16384 records
-    bp.m = (bp.E * kBucketNT) / kBucketStride - bp.runs;  // (m + runs) G = capacity
+    for (int j = 0; j < bp.runs; ++j) bp.samples += run_len(cols, bp.chunk, j) / bp.G;
+    bp.m = bp.cap / bp.G - bp.runs;  // (m + runs) G = capacity
+    // few rows: smaller buckets, so that they fill the chip once
+    const int64_t want = ((int64_t)256 * (16384 / bp.cap) + rows - 1) / rows;
+    int64_t fine = (bp.samples + want - 1) / want;
+    // ... but at most about two searches per thread of the splitter kernel
+    const int64_t least = ((int64_t)bp.samples * bp.runs + 2 * kSplitNT - 1) / (2 * kSplitNT);
+    fine = fine < least ? least : fine;
+    if (fine < bp.m) bp.m = fine < 8 ? 8 : (int)fine;
     bp.K = (bp.samples + bp.m - 1) / bp.m;
     if (bp.K < 1) bp.K = 1;
     if (rows * bp.K > 2147483647) {
@@ -801,18 +974,10 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
     hipLaunchKernelGGL(bucket_split_kernel, dim3((unsigned)rows), dim3(kSplitNT), 0, s, a, bp, buf[0], table);
     st = launch_status("tallax_sort_rows (splitters)");
     if (st) return st;
-    const int lds = bp.E * kBucketNT * 8 + 256 * (kBucketNT / kWave + 1) * 4;
-    const void* kfn = bp.E == 16 ? (const void*)bucket_sort_kernel<16> : (const void*)bucket_sort_kernel<32>;
-    const hipError_t attr = set_dynamic_lds_limit(kfn, lds, s);
-    if (attr != hipSuccess) {
-      set_error("hipFuncSetAttribute: %s", hipGetErrorString(attr));
-      return kHipError;
-    }
-    const dim3 grid((unsigned)(rows * bp.K));
-    if (bp.E == 16)
-      hipLaunchKernelGGL(bucket_sort_kernel<16>, grid, dim3(kBucketNT), lds, s, a, bp, (const uint64_t*)buf[0], table);
-    else
-      hipLaunchKernelGGL(bucket_sort_kernel<32>, grid, dim3(kBucketNT), lds, s, a, bp, (const uint64_t*)buf[0], table);
+    const int st2 = a.key_dtype == kBF16 ? launch_buckets<kBF16>(a, rows, bp, buf[0], table, s)
+                    : a.key_dtype == kI32 ? launch_buckets<kI32>(a, rows, bp, buf[0], table, s)
+                                          : launch_buckets<kF32>(a, rows, bp, buf[0], table, s);
+    if (st2) return st2;
     return launch_status("tallax_sort_rows (buckets)");
   }
   const int passes = wide_passes(cols);

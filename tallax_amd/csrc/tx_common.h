@@ -180,6 +180,16 @@ __device__ __forceinline__ int wave_max_i(int v) {
   return max(v, (int)lane_xor((uint32_t)v, 1));
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, lane_xor(v, 32));
+  v = max(v, lane_xor(v, 16));
+  v = max(v, lane_xor(v, 8));
+  v = max(v, lane_xor(v, 4));
+  v = max(v, lane_xor(v, 2));
+  return max(v, lane_xor(v, 1));
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) { return ~wave_max_u32(~v); }
+
 __device__ __forceinline__ uint32_t wave_and_u32(uint32_t v) {
   v &= lane_xor(v, 32);
   v &= lane_xor(v, 16);
