@@ -28,6 +28,8 @@ MAX_WIDE_CANDIDATES = 1024  # widest opt-in candidate list (tallax_sample_wide)
 
 def _key_tensor(rng_key: Any, device: torch.device) -> torch.Tensor:
     if isinstance(rng_key, torch.Tensor):
+        if rng_key.dtype is torch.int32 and rng_key.shape == (2,) and rng_key.device == device:
+            return rng_key.contiguous()
         k = rng_key.reshape(-1)
         if k.numel() != 2:
             raise ValueError(f"rng_key must hold 2 uint32 words, got {k.numel()}")
@@ -42,6 +44,9 @@ def _key_tensor(rng_key: Any, device: torch.device) -> torch.Tensor:
 
 
 def _per_row(v: Any, rows: int, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    # what a serving loop passes: its own device tensor, used as it is
+    if isinstance(v, torch.Tensor) and v.dtype is dtype and v.shape == (rows,) and v.device == device:
+        return v.contiguous()
     if isinstance(v, numbers.Number):
         # filled on the device: no host-to-device copy, so the call can be graph-captured
         return torch.full((rows,), v, dtype=dtype, device=device)

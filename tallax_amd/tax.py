@@ -145,7 +145,8 @@ def _top_dynamic_k(logits, k, max_k, block_token, num_bins, bins_topm_unroll, bi
         _lib.check(_lib.LIB.tallax_testing_top_dynamic_k_path(*args, int(testing_path)), "top_dynamic_k")
     if guarantee_convergence:
         return vals, idx
-    return vals, idx, valid.reshape(()).bool(), depths, cutoff
+    # the low byte of the 0 / 1 word, as a view: no conversion launch
+    return vals, idx, valid.view(torch.bool)[0], depths, cutoff
 
 
 _SORT_DTYPES = (torch.float32, torch.bfloat16, torch.int32)
@@ -178,14 +179,19 @@ def sort(operand, num_keys: int, is_stable: bool = False, return_argsort: bool =
     accepted and ignored.
     """
     del num_vmem_substages, block_token, interpret
+    return _sort(operand, num_keys, is_stable, return_argsort, descending)
+
+
+def _sort(operand, num_keys, is_stable, return_argsort, descending, want_key: bool = True) -> tuple:
+    """sort; with want_key=False the first key's sorted values are neither
+    written nor returned (None in their place)."""
     operands = list(operand) if isinstance(operand, (list, tuple)) else [operand]
     if not operands:
         raise ValueError("sort needs at least one operand")
     _lib.require_cuda(*operands)
-    shapes = {tuple(x.shape) for x in operands}
-    if len(shapes) != 1:
+    shape = operands[0].shape
+    if any(x.shape != shape for x in operands[1:]):
         raise ValueError(f"Inputs must all have the same shape, but found shapes={[tuple(x.shape) for x in operands]}")
-    shape = shapes.pop()
     if len(shape) != 2:
         raise ValueError("Only 2D inputs supported")
     num_keys = int(num_keys)
@@ -213,7 +219,8 @@ def sort(operand, num_keys: int, is_stable: bool = False, return_argsort: bool =
     perm = torch.empty(shape, dtype=torch.int32, device=dev)
     outs = [None] * len(ops)
     k0 = ops[0]
-    out0 = torch.empty(shape, dtype=key_out_dtype(k0), device=dev)
+    out0 = torch.empty(shape, dtype=key_out_dtype(k0), device=dev) if want_key else None
+    out0_ptr, out0_dt = (out0.data_ptr(), _lib.dtype_code(out0)) if want_key else (None, 0)
     # rows longer than 16384: a per-call workspace (the caching allocator recycles it)
     nws = int(_lib.LIB.tallax_sort_rows_workspace_size(rows, cols))
     ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws else None
@@ -221,7 +228,7 @@ def sort(operand, num_keys: int, is_stable: bool = False, return_argsort: bool =
     if num_keys == 1:
         _lib.check(_lib.LIB.tallax_sort_rows_ws(
             k0.data_ptr(), _lib.dtype_code(k0), rows, cols, int(bool(descending)), int(ties_desc), None,
-            perm.data_ptr(), out0.data_ptr(), _lib.dtype_code(out0), None, 0, None, 0, ws_ptr, nws, stream), "sort")
+            perm.data_ptr(), out0_ptr, out0_dt, None, 0, None, 0, ws_ptr, nws, stream), "sort")
     else:
         # stable LSD passes, last key first; each pass sorts key[perm] with
         # position ties and composes, so the final permutation orders the rows
@@ -239,7 +246,7 @@ def sort(operand, num_keys: int, is_stable: bool = False, return_argsort: bool =
         out1 = torch.empty(shape, dtype=key_out_dtype(k1), device=dev)
         _lib.check(_lib.LIB.tallax_sort_rows_ws(
             k0.data_ptr(), _lib.dtype_code(k0), rows, cols, int(bool(descending)), 0, prev.data_ptr(),
-            perm.data_ptr(), out0.data_ptr(), _lib.dtype_code(out0), k1.data_ptr(), _lib.dtype_code(k1),
+            perm.data_ptr(), out0_ptr, out0_dt, k1.data_ptr(), _lib.dtype_code(k1),
             out1.data_ptr(), _lib.dtype_code(out1), ws_ptr, nws, stream), "sort")
         outs[1] = out1
         for i in range(2, num_keys):  # further keys: gathered by the final permutation, decoded like keys

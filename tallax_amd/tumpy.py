@@ -18,6 +18,8 @@ def _rows_view(a: torch.Tensor, axis):
     canonical = axis if axis >= 0 else axis + ndim
     if canonical != ndim - 1:
         raise ValueError("tumpy only supports sorting along the last axis.")
+    if ndim == 2:
+        return a, a.shape
     return a.reshape(-1, a.shape[-1]), tuple(a.shape)
 
 
@@ -32,7 +34,7 @@ def sort(a: torch.Tensor, axis=-1, kind=None, order=None, stable: bool = True, d
     from . import tax
     a2, shape = _rows_view(a, axis)
     (out,) = tax.sort(a2, num_keys=1, is_stable=stable, descending=descending, return_argsort=False)
-    return out.reshape(shape)
+    return out if out.shape == shape else out.reshape(shape)
 
 
 def argsort(a: torch.Tensor, axis=-1, kind=None, order=None, stable: bool = True, descending: bool = False,
@@ -45,8 +47,8 @@ def argsort(a: torch.Tensor, axis=-1, kind=None, order=None, stable: bool = True
     del kind, order, interpret
     from . import tax
     a2, shape = _rows_view(a, axis)
-    _, idx = tax.sort(a2, num_keys=1, is_stable=stable, descending=descending, return_argsort=True)
-    return idx.reshape(shape)
+    _, idx = tax._sort(a2, 1, stable, True, descending, want_key=False)  # the sorted keys are not written
+    return idx if idx.shape == shape else idx.reshape(shape)
 
 
 def take_along_axis(arr: torch.Tensor, indices: torch.Tensor, axis: int, interpret: bool = False) -> torch.Tensor:
@@ -71,7 +73,7 @@ def take_along_axis(arr: torch.Tensor, indices: torch.Tensor, axis: int, interpr
     if arr.shape[other] != indices.shape[other]:
         raise ValueError(f"batch extents differ: {tuple(arr.shape)} vs {tuple(indices.shape)} along axis {other}")
     x = arr.contiguous()
-    idx = indices.to(torch.int32).contiguous()
+    idx = (indices if indices.dtype is torch.int32 else indices.to(torch.int32)).contiguous()
     dt = _lib.dtype_code(x)
     out = torch.empty(idx.shape, dtype=x.dtype, device=x.device)
     _lib.check(_lib.LIB.tallax_take_along_axis(x.data_ptr(), dt, x.shape[0], x.shape[1], idx.data_ptr(),
