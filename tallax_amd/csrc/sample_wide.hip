@@ -39,8 +39,9 @@
 // The row is read two (bf16) to four (f32) times; the re-reads of a row just
 // streamed are served mostly from the caches.
 //
-// Rows of whole 16-byte vectors that fit 16 vectors per thread (bf16 up to
-// 131072 columns, f32 up to 65536) take a single read first: the vectors stay
+// Rows that fit 19 vectors per thread (bf16 up to 155648 columns, f32 up to
+// 77824, less a few where the row is not whole aligned vectors) take a single
+// read first: the vectors stay
 // in registers; each lane keeps its four largest vector maxima (integer max
 // over the raw bits, which orders non-negative values), each wave takes the
 // ceil(K / 16)-th largest of its 256 kept maxima, and L, the smallest of those
@@ -184,7 +185,12 @@ __device__ __forceinline__ void sw_cross(const int* hist, int need, int* red, in
   __syncthreads();
 }
 
-template <int DT>
+// EDGE: rows that do not start 16-byte aligned or do not fill their last vector.
+// The register path reads them as whole aligned vectors too; the slots of the
+// first and last one outside the row become all-ones ([37, 47070] f32,
+// K = 512, on the element loads of the radix select before: 57 -> 22 us,
+// [18, 110978] bf16 K = 1024 71 -> 24).
+template <int DT, bool EDGE>
 __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
   constexpr int ES = DT == kBF16 ? 2 : 4;
   __shared__ int s_hist[kSwBins];
@@ -222,15 +228,39 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
   // --- register path: one read, the elements >= L -----------------------------
   constexpr int VEC = DT == kBF16 ? 8 : 4;
   constexpr int32_t kPosInf = DT == kBF16 ? 0x7F80 : 0x7F800000;  // +inf bits in the signed view
-  const int64_t nvec = a.cols / VEC;  // a.vec: the row is whole 16-byte vectors
-  bool fast = vec && nvec <= (int64_t)kSwNT * kSwV;  // block-uniform
+  const RowVec<ES> rv(rowp);
+  const int mis = EDGE ? rv.mis : 0;  // slots of the first vector before the row
+  const int64_t nvec = (a.cols + mis + VEC - 1) / VEC;
+  bool fast = nvec <= (int64_t)kSwNT * kSwV;  // block-uniform
   if (fast) {
-    const uint4* vb = (const uint4*)rowp;
+    const uint4* vb = EDGE ? rv.base : (const uint4*)rowp;
     uint4 raw[kSwV];
 #pragma unroll
     for (int j = 0; j < kSwV; ++j) {
       const int64_t v = (int64_t)j * kSwNT + t;
       raw[j] = v < nvec ? load_once(vb + v) : make_uint4(~0u, ~0u, ~0u, ~0u);  // all-ones: -1, below every bound
+    }
+    if (EDGE) {
+      const int tail = (int)(a.cols + mis - (nvec - 1) * VEC);  // live slots of the last vector, 1..VEC
+      if (mis > 0 || tail < VEC) {
+        // one thread may own both vectors, as different ones
+        int hj = t == 0 && mis > 0 ? 0 : -1, tj = -1, lo = mis, hi = tail;
+        if (t == (int)((nvec - 1) % kSwNT) && tail < VEC) tj = (int)((nvec - 1) / kSwNT);
+        // the empty asm keeps the masks derived from these values in this block
+        asm volatile("" : "+v"(hj), "+v"(tj), "+v"(lo), "+v"(hi));
+#pragma unroll
+        for (int j = 0; j < kSwV; ++j) {
+          uint32_t d[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+          const int l0 = hj == j ? lo : 0, h0 = tj == j ? hi : VEC;
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            const bool dead = e < l0 || e >= h0;
+            if (DT == kBF16) d[e >> 1] |= dead ? ((e & 1) ? 0xFFFF0000u : 0x0000FFFFu) : 0u;
+            else d[e] |= dead ? ~0u : 0u;
+          }
+          raw[j] = make_uint4(d[0], d[1], d[2], d[3]);
+        }
+      }
     }
     if (t == 0) s_cnt = 0;
     // this lane's four largest vector maxima; a positive NaN maximum sends the row to the radix select
@@ -311,7 +341,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
           const int o = wcnt + (int)__popcll(b & ((1ull << l) - 1ull));
           if (f && o < kSwStage) {
             s_vst[w][o] = raw[j];
-            s_vcol[w][o] = (uint32_t)(((int64_t)j * kSwNT + t) * VEC);
+            s_vcol[w][o] = (uint32_t)((j * kSwNT + t) * VEC - mis);
           }
           wcnt += (int)__popcll(b);
         }
@@ -364,7 +394,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
         for (int j = 0; j < kSwV; ++j) {
           const uint32_t m = (pm[j >> 2] >> (8 * (j & 3))) & 0xFFu;
           if (!__ballot(m != 0u)) continue;  // wave-uniform
-          put(raw[j], m, (uint32_t)(((int64_t)j * kSwNT + t) * VEC), pos);
+          put(raw[j], m, (uint32_t)((j * kSwNT + t) * VEC - mis), pos);
           pos += __popc(m);
         }
       }
@@ -683,9 +713,11 @@ int tallax_sample_wide(const void* logits, int dtype, int64_t rows, int64_t voca
   a.replace_in_dtype = dtype == kBF16 ? round_to_bf16(rf) : rf;
   a.out_tokens = out_tokens; a.out_idx = out_idx; a.out_vals = out_vals;
   if (dtype == kF32)
-    sample_wide_kernel<kF32><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
+    a.vec ? sample_wide_kernel<kF32, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
+          : sample_wide_kernel<kF32, true><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
   else
-    sample_wide_kernel<kBF16><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
+    a.vec ? sample_wide_kernel<kBF16, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
+          : sample_wide_kernel<kBF16, true><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
   return launch_status("tallax_sample_wide");
 }
 
