@@ -501,9 +501,14 @@ __global__ __launch_bounds__(256) void cumsum_col_tiles_kernel(const T* __restri
 // lines (a power of two <= 64); all its threads stage a block of totals into
 // LDS (16 loads in flight per thread; line_major: consecutive threads on
 // consecutive tiles of a line, else on consecutive lines), lane j of wave 0
-// chains line j from LDS (line-major rows, 16-byte reads and writes, 32 adds
-// per stretch with no branch: one dependent add per tile), and all threads
-// store the block's final values.
+// chains line j from LDS (line-major rows, 16-byte reads, 32 adds per stretch
+// with no branch: one dependent add per tile) and keeps only each stretch's
+// start, then all threads repeat the stretches from there and store the
+// block's final values.  The serial lane writes one word per 32 adds: a lane
+// that reads and writes every total takes 8.3 ns per add, against 4.3 with the
+// reads alone and 2.0 for the dependent add (f32 [1, 4000000] 275 -> 203 us,
+// [8, 1000000] 93 -> 75, [128256, 8] axis 0 147 -> 109, [64, 128257] 38.8 -> 36.7;
+// the rest is the LDS reads' issue).
 constexpr int kChainNT = 256;
 constexpr int kChainBuf = 16384;  // LDS words (64 KiB for 4-byte T)
 constexpr int kChainRun = 32;     // tiles per branch-free stretch of the chain
@@ -519,7 +524,8 @@ __global__ __launch_bounds__(kChainNT) void cumsum_chain_kernel(T* __restrict__ 
                                                                 int64_t step, int ts, int64_t plen, int reverse,
                                                                 int64_t ntot, int gl, int line_major) {
   static_assert(sizeof(T) == 4, "4-byte totals");
-  __shared__ __align__(16) T buf[kChainBuf];  // buf[line * rs + t]
+  __shared__ __align__(16) T buf[kChainBuf + 2 * kChainRun];  // buf[line * rs + t]; two stretches read past the last line
+  __shared__ T start[kChainBuf / kChainRun];                  // running total before each stretch, [line][stretch]
   const int64_t L0 = (int64_t)blockIdx.x * gl;
   const int tb = kChainBuf / gl - kChainRun;  // tiles per block, a multiple of kChainRun
   const int rs = tb + 4;                       // LDS row stride (16-byte aligned, staggered banks)
@@ -548,27 +554,62 @@ __global__ __launch_bounds__(kChainNT) void cumsum_chain_kernel(T* __restrict__ 
       }
     }
     __syncthreads();
-    if (j0 < gl) {
-      // stretches past nb read and rewrite LDS words that are never stored
-      // to memory; acc is then spent (only the last block is partial)
-      uint4* row = (uint4*)(buf + j0 * rs);
-      for (int i0 = 0; i0 < nb; i0 += kChainRun) {
-        uint4 q[kChainRun / 4];
+    const int ns = (nb + kChainRun - 1) / kChainRun;  // stretches of a line
+    if (ns == 1) {  // at most 32 tiles, the line's only block: the repeat below is the chain
+      if (j0 < gl) start[j0] = acc;
+    } else if (j0 < gl) {
+      // the running total before each stretch: one dependent add per tile, the
+      // next stretch's LDS reads in flight meanwhile.  A partial stretch reads
+      // LDS words past nb; acc is then spent (only the last block is partial).
+      constexpr int Q = kChainRun / 4;
+      const uint4* row = (const uint4*)(buf + j0 * rs);
+      T* cr = start + j0 * ns;
+      // a stretch past the line's last one reads words that are never used
+      auto load = [&](int i, uint4 (&q)[Q]) {
 #pragma unroll
-        for (int u = 0; u < kChainRun / 4; ++u) q[u] = row[i0 / 4 + u];
+        for (int u = 0; u < Q; ++u) q[u] = row[i * Q + u];
+        __builtin_amdgcn_sched_barrier(0);  // the reads go out before the adds of the stretch at hand
+      };
+      auto chain = [&](const uint4 (&q)[Q]) {
 #pragma unroll
-        for (int u = 0; u < kChainRun / 4; ++u) {
+        for (int u = 0; u < Q; ++u) {
           acc = add_in_order(__builtin_bit_cast(T, q[u].x), acc);
-          q[u].x = __builtin_bit_cast(uint32_t, acc);
           acc = add_in_order(__builtin_bit_cast(T, q[u].y), acc);
-          q[u].y = __builtin_bit_cast(uint32_t, acc);
           acc = add_in_order(__builtin_bit_cast(T, q[u].z), acc);
-          q[u].z = __builtin_bit_cast(uint32_t, acc);
           acc = add_in_order(__builtin_bit_cast(T, q[u].w), acc);
-          q[u].w = __builtin_bit_cast(uint32_t, acc);
         }
+      };
+      uint4 q0[Q], q1[Q];
+      load(0, q0);
+      for (int i = 0; i < ns; i += 2) {
+        load(i + 1, q1);
+        cr[i] = acc;
+        chain(q0);
+        if (i + 1 >= ns) break;
+        load(i + 2, q0);
+        cr[i + 1] = acc;
+        chain(q1);
+      }
+    }
+    __syncthreads();
+    // every stretch again, from its own start, by a thread of its own: the same
+    // adds in the same order, this time writing each final value
+    for (int e = j0; e < gl * ns; e += kChainNT) {
+      const int ll = e / ns, i = e - ll * ns;
+      uint4* q = (uint4*)(buf + ll * rs) + i * (kChainRun / 4);
+      T f = start[e];
 #pragma unroll
-        for (int u = 0; u < kChainRun / 4; ++u) row[i0 / 4 + u] = q[u];
+      for (int u = 0; u < kChainRun / 4; ++u) {
+        uint4 x = q[u];
+        f = add_in_order(__builtin_bit_cast(T, x.x), f);
+        x.x = __builtin_bit_cast(uint32_t, f);
+        f = add_in_order(__builtin_bit_cast(T, x.y), f);
+        x.y = __builtin_bit_cast(uint32_t, f);
+        f = add_in_order(__builtin_bit_cast(T, x.z), f);
+        x.z = __builtin_bit_cast(uint32_t, f);
+        f = add_in_order(__builtin_bit_cast(T, x.w), f);
+        x.w = __builtin_bit_cast(uint32_t, f);
+        q[u] = x;
       }
     }
     __syncthreads();

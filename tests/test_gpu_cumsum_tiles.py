@@ -43,3 +43,18 @@ def test_cumsum_unaligned_view(gpu):
     x = buf[1:].view(3, 9001)
     got = tax.cumsum(x, 1).cpu().numpy()
     assert np.array_equal(bits(got), bits(O.cumsum(x.cpu().numpy(), 1)))
+
+
+# the chain's stretches of 32 totals: one, a partial second, both of a pair of
+# stretches and one more, several lines per workgroup, more than one staged block
+@pytest.mark.parametrize("shape,axis", [((33 * 8 + 3, 5), 0), ((34 * 8, 5), 0), ((65 * 8 + 1, 700), 0),
+                                        ((97 * 8, 1100), 0), ((1, 128 * 4200), 1), ((20000, 129 * 8), 0),
+                                        ((1, 128 * 16400), 1)])
+@pytest.mark.parametrize("reverse", [False, True])
+def test_cumsum_chain_stretches(gpu, shape, axis, reverse):
+    from tallax_amd import tax
+    print(f"cumsum chain {shape} axis={axis} reverse={reverse}", flush=True)
+    rng = np.random.default_rng(shape[0] + shape[1])
+    x = rng.standard_normal(shape).astype(np.float32)
+    got = tax.cumsum(torch.from_numpy(x).to(gpu), axis, reverse=reverse).cpu().numpy()
+    assert np.array_equal(bits(got), bits(O.cumsum(x, axis, reverse)))
