@@ -117,10 +117,60 @@ __device__ __forceinline__ int pf_crossing_bin(const uint32_t* h, uint32_t need,
   return b;
 }
 
+// The k-th largest composite of a row by a radix select over its 8-bit digits,
+// one read of the row per digit, until the crossing bin is taken whole: two to
+// four reads where few values tie, eight at most (a bisection read the row 64
+// times: [2, 10926] k = 1616 141 -> 40 us, [300, 16384] k = 2048 305 -> 80,
+// [16, 25000] 268 -> 58).  hist: 256 counters, res: 3 words of LDS.  Every
+// thread of the workgroup calls it.
+__device__ __attribute__((noinline)) uint64_t pf_kth_comp(const uint4* base, int64_t nv, int mis, int64_t cols, int k,
+                                                          uint32_t* hist, int* res) {
+  const int t = threadIdx.x;
+  uint64_t prefix = 0;
+  int need = k;
+#pragma unroll 1
+  for (int sh = 56; sh >= 0; sh -= 8) {
+    if (t < 256) hist[t] = 0u;
+    __syncthreads();
+#pragma unroll 1
+    for (int64_t v = t; v < nv; v += kPfNT) {
+      const uint4 q = base[v];
+      const uint32_t d[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t e = v * 4 - mis + i;
+        const uint64_t c = make_comp(select_key(d[i]), (uint32_t)e);
+        if (e >= 0 && e < cols && (sh == 56 || ((c ^ prefix) >> (sh + 8)) == 0ull))
+          atomicAdd(&hist[(uint32_t)(c >> sh) & 255u], 1u);
+      }
+    }
+    __syncthreads();
+    if (t < kWave) {
+      uint32_t above;
+      const int b = pf_crossing_bin(hist, (uint32_t)need, &above);  // >= 0: the row has at least k elements
+      if (t == 0) {
+        res[0] = b;
+        res[1] = (int)above;
+        res[2] = (int)hist[b];
+      }
+    }
+    __syncthreads();
+    prefix |= (uint64_t)(uint32_t)res[0] << sh;
+    need -= res[1];
+    if (res[2] == need) break;  // block-uniform
+  }
+  __syncthreads();
+  return prefix;
+}
+
 // 8 waves per SIMD: two row workgroups share a CU, so one streams while the
 // other sorts.  SUMM: group summary and histogram threshold (rows of at most
 // kPfMaxGroups groups); otherwise per-thread top-4 and a full second read.
-template <bool SUMM>
+// SHORT: rows whose groups are too few to bound the candidates (the launch's
+// rule); every such row takes pf_kth_comp.  The other instances keep the
+// bisection for rows of heavy ties: a call there costs the streaming loop
+// registers ([1024, 201088] 194 -> 202 us, 207 inlined).
+template <bool SUMM, bool SHORT>
 __global__ __launch_bounds__(kPfNT) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void softmax_topk_kernel(PfArgs a) {
   extern __shared__ __align__(16) uint64_t pool[];  // a.cap records, then the group maxima / list / probabilities
@@ -637,27 +687,31 @@ void softmax_topk_kernel(PfArgs a) {
     else if (n <= 4 * kPfNT) pf_sort_desc<4>(pool, n);
     else pf_sort_desc<8>(pool, n);
   } else {
-    // heavy ties: bisection for the k-th largest composite over the row
     uint64_t prefix = 0;
-    for (int bit = 63; bit >= 0; --bit) {
-      const uint64_t probe = prefix | (1ull << bit);
-      int c = 0;
-      for (int64_t v = t; v < nv; v += kPfNT) {
-        const uint4 q = rv.base[v];
-        const uint32_t d[4] = {q.x, q.y, q.z, q.w};
+    if constexpr (SHORT) {
+      prefix = pf_kth_comp(rv.base, nv, rv.mis, a.cols, k, hist, redi);
+    } else {
+      // heavy ties: bisection for the k-th largest composite over the row
+      for (int bit = 63; bit >= 0; --bit) {
+        const uint64_t probe = prefix | (1ull << bit);
+        int c = 0;
+        for (int64_t v = t; v < nv; v += kPfNT) {
+          const uint4 q = rv.base[v];
+          const uint32_t d[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int64_t e = v * 4 - rv.mis + i;
-          if (e >= 0 && e < a.cols) c += make_comp(select_key(d[i]), (uint32_t)e) >= probe;
+          for (int i = 0; i < 4; ++i) {
+            const int64_t e = v * 4 - rv.mis + i;
+            if (e >= 0 && e < a.cols) c += make_comp(select_key(d[i]), (uint32_t)e) >= probe;
+          }
         }
+        c = wave_sum_i(c);
+        __syncthreads();
+        if (l == 0) redi[w] = c;
+        __syncthreads();
+        int tot = 0;
+        for (int i = 0; i < kPfNW; ++i) tot += redi[i];
+        if (tot >= k) prefix = probe;
       }
-      c = wave_sum_i(c);
-      __syncthreads();
-      if (l == 0) redi[w] = c;
-      __syncthreads();
-      int tot = 0;
-      for (int i = 0; i < kPfNW; ++i) tot += redi[i];
-      if (tot >= k) prefix = probe;
     }
     if (t == 0) s_cnt = 0;
     __syncthreads();
@@ -776,16 +830,25 @@ int tallax_softmax_topk_cumsum(const float* logits, int64_t rows, int64_t cols, 
   a.cap = cap;
   a.cap2 = (int)(region2 / 8);
   const size_t lds = (size_t)cap * 8 + region2;
-  const hipError_t attr1 = set_dynamic_lds_limit((const void*)softmax_topk_kernel<true>, kPfDynBytes, stream);
-  const hipError_t attr0 = set_dynamic_lds_limit((const void*)softmax_topk_kernel<false>, kPfDynBytes, stream);
-  if (attr1 != hipSuccess || attr0 != hipSuccess) {
-    set_error("hipFuncSetAttribute: %s", hipGetErrorString(attr1 != hipSuccess ? attr1 : attr0));
+  // Fewer than 1.25 k groups: the k-th group maximum leaves more candidates
+  // than the pool's 2 k or so (normal logits: 10 % of 20 k elements), so the
+  // row needs the exact threshold.
+  const bool is_short = summ && ngroups * 4 < (int64_t)k * 5;
+  const void* kern = !summ      ? (const void*)softmax_topk_kernel<false, false>
+                     : is_short ? (const void*)softmax_topk_kernel<true, true>
+                                : (const void*)softmax_topk_kernel<true, false>;
+  const hipError_t attr = set_dynamic_lds_limit(kern, kPfDynBytes, stream);
+  if (attr != hipSuccess) {
+    set_error("hipFuncSetAttribute: %s", hipGetErrorString(attr));
     return kHipError;
   }
-  if (summ)
-    hipLaunchKernelGGL(softmax_topk_kernel<true>, dim3((unsigned)rows), dim3(kPfNT), lds, stream, a);
+  const dim3 grid((unsigned)rows), block(kPfNT);
+  if (!summ)
+    hipLaunchKernelGGL((softmax_topk_kernel<false, false>), grid, block, lds, stream, a);
+  else if (is_short)
+    hipLaunchKernelGGL((softmax_topk_kernel<true, true>), grid, block, lds, stream, a);
   else
-    hipLaunchKernelGGL(softmax_topk_kernel<false>, dim3((unsigned)rows), dim3(kPfNT), lds, stream, a);
+    hipLaunchKernelGGL((softmax_topk_kernel<true, false>), grid, block, lds, stream, a);
   return launch_status("tallax_softmax_topk_cumsum");
 }
 
