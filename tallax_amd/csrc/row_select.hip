@@ -69,6 +69,9 @@ constexpr int kUnevenMaxBlocks = 256;      // at least half of the CUs (plan_row
 struct SelArgs {
   const void* x;
   int64_t rows, cols;
+  // what the whole-row kernel's first loads wait for stays in the arguments' first 64 bytes
+  int part_cols;        // whole-row kernel: part p of a row holds columns [p * part_cols, (p + 1) * part_cols)
+  int list_k;           // whole-row kernel: places of the row's (or part's) list that are read (64; 0: all 128)
   int k;
   int nseg;
   int64_t vps;  // 16-byte vectors per segment
@@ -80,8 +83,6 @@ struct SelArgs {
   uint64_t* ws_lists;
   int lists_only;  // write the segment list even when a row is one segment
   int64_t col_offset;   // added to every column index of a written list (a vocabulary shard's first column)
-  int part_cols;        // whole-row kernel: part p of a row holds columns [p * part_cols, (p + 1) * part_cols)
-  int list_k;           // whole-row kernel: places of the row's (or part's) list that are read (64; 0: all 128)
   uint64_t* out_lists;  // merge kernel, lists_only: the merged list of each row, [rows][128]
   // sampler
   const int32_t* top_k;
@@ -1346,10 +1347,12 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   __shared__ SegShared<CT, kNTS> sh;  // tie path, output list
   __shared__ uint4 stage[2 * kNTS];   // tie path
   const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
-  const int64_t row = blockIdx.x;
-  // row parts (SAMPLE = false only): workgroup (row, part) of a two-dimensional
-  // grid; the row's last part may be shorter (part_cols = cols: whole rows)
-  const int64_t c0 = SAMPLE ? 0 : (int64_t)((uint64_t)blockIdx.y * (uint32_t)a.part_cols);
+  // row parts (SAMPLE = false only): workgroup (part, row) of a two-dimensional
+  // grid, so that a row's parts run side by side; its last part may be shorter
+  const bool parts = !SAMPLE && a.part_cols < a.cols;
+  const int64_t row = parts ? blockIdx.y : blockIdx.x;
+  const unsigned part = parts ? blockIdx.x : 0u;
+  const int64_t c0 = (int64_t)((uint64_t)part * (uint32_t)a.part_cols);
   const int left = (int)(a.cols - c0), cols = SAMPLE || left < a.part_cols ? left : a.part_cols;
   const char* rowp = (const char*)a.x + (size_t)(row * a.cols + c0) * ES;
   const RowVec<ES> rv(rowp);
@@ -1656,7 +1659,7 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   if (!a.lists_only) {
     finalize_row<DT, SAMPLE>(a, row, sh.list64, sh.samp_g, rp);
   } else {
-    uint64_t* dst = a.ws_lists + (size_t)(row * gridDim.y + blockIdx.y) * kRun;
+    uint64_t* dst = a.ws_lists + (size_t)(parts ? row * gridDim.x + part : row) * kRun;
     const uint64_t off = (uint64_t)(a.col_offset + c0);
     for (int i = tid; i < kq; i += kNTS) dst[i] = sh.list64[i] ? sh.list64[i] - off : 0ull;
   }
@@ -1862,7 +1865,7 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
     // (the row's last part too: cols and part_cols both are whole vectors)
     const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0 ||
                       ((int64_t)a.part_cols * ElemT<DT>::ES) % 16 != 0;
-    const dim3 g((unsigned)a.rows, (unsigned)p.parts), b(kNTS);
+    const dim3 g((unsigned)p.parts, (unsigned)a.rows), b(kNTS);
     if (p.maxv == 19) {
       if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true>), g, b, 0, s, a);
       else hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, false>), g, b, 0, s, a);
