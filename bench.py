@@ -636,7 +636,7 @@ def _sort_wide(torch, np, _lib, dev, s_handle, gen, nbuf):
     w.workload = ("tax.sort(p, num_keys=1, is_stable=True, return_argsort=True, descending=True) of f32 "
                   "[1024,201088] softmax(N(0, sigma=2)) rows: the reference's sort route for config 5 "
                   "(rows > 16384: chunk radix sorts, then a multiway merge by splitters through the workspace)")
-    w.kernel = "sort_chunks_kernel<f32> + bucket_split_kernel + bucket_sort_kernel<16>"
+    w.kernel = "sort_chunks_kernel<f32> + bucket_split_kernel + bucket_sort_kernel<256, 16>"
     w.cpu_batch = 1
     sample = 4  # rows checked against the oracle
 
