@@ -64,6 +64,7 @@ _SIGNATURES = {
     "tallax_testing_read_bytes": ([_c_p, _c_i64, _c_int, _c_p, _c_p], _c_int),
     "tallax_testing_lds_atomic_order": ([_c_p, _c_i64, _c_int, _c_p, _c_p], _c_int),
     "tallax_testing_select_plan": ([_c_i64, _c_i64, _c_int, _c_p], _c_int),
+    "tallax_testing_select_edge": ([_c_i64, _c_i64, _c_int, _c_p], _c_int),
     "tallax_testing_top_dynamic_k_path": ([_c_p, _c_int, _c_i64, _c_i64, _c_p, _c_int, _c_int, _c_int, _c_p, _c_int,
                                            _c_int, _c_int, _c_d, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_sz, _c_p, _c_int],
                                           _c_int),
@@ -194,7 +195,8 @@ def select_plan(rows: int, cols: int, dtype: int, k: int = 128, sample: bool = T
         else "seg_merge_kernel"
     if nt == 1024:
         # EDGE: rows (or parts) not a whole number of 16-byte vectors (a 16-byte aligned base assumed)
-        edge = "true" if (cols // nseg * (4 if dtype == F32 else 2)) % 16 else "false"
+        check(LIB.tallax_testing_select_edge(rows, cols, dtype, out), "select_plan")
+        edge = "true" if out[0] else "false"
         if nseg == 1:
             name = f"stream_select_kernel<{dt}, {maxv}, SAMPLE, {edge}>"
         else:

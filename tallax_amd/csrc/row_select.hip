@@ -1771,6 +1771,13 @@ static int64_t part_cols_of(int64_t cols, int np, int vec) {
   return (per + vec - 1) / vec * vec;
 }
 
+// EDGE instance of the whole-row kernel: some row or part does not start
+// 16-byte aligned or does not fill its last vector (a row's last part too:
+// where cols and part_cols both are whole vectors, it is as well).
+static bool whole_row_edge(const void* x, int64_t cols, int64_t part_cols, int es) {
+  return ((uintptr_t)x % 16) != 0 || (cols * es) % 16 != 0 || (part_cols * es) % 16 != 0;
+}
+
 static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
   const int vec = dt == kF32 ? 4 : 8;
   const int64_t nv = (cols + 2 * (vec - 1)) / vec;  // covers any row misalignment
@@ -1861,10 +1868,7 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
   }
   const SelArgs& a = h;
   if (p.nt == kNTS && p.parts > 1) {
-    // every row and every part starts 16-byte aligned and fills its last vector
-    // (the row's last part too: cols and part_cols both are whole vectors)
-    const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0 ||
-                      ((int64_t)a.part_cols * ElemT<DT>::ES) % 16 != 0;
+    const bool edge = whole_row_edge(a.x, a.cols, a.part_cols, ElemT<DT>::ES);
     const dim3 g((unsigned)p.parts, (unsigned)a.rows), b(kNTS);
     if (p.maxv == 19) {
       if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true>), g, b, 0, s, a);
@@ -1874,9 +1878,7 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
       else hipLaunchKernelGGL((stream_select_kernel<DT, 16, false, false>), g, b, 0, s, a);
     }
   } else if (p.nt == kNTS) {
-    // rows that start 16-byte aligned and fill their last vector have no
-    // slots outside the row: the kernel without the edge handling
-    const bool edge = ((uintptr_t)a.x % 16) != 0 || (a.cols * ElemT<DT>::ES) % 16 != 0;
+    const bool edge = whole_row_edge(a.x, a.cols, a.cols, ElemT<DT>::ES);
     const dim3 g((unsigned)a.rows), b(kNTS);
     if (p.maxv == 19) {
       if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, SAMPLE, true>), g, b, 0, s, a);
@@ -2339,6 +2341,19 @@ int tallax_testing_select_plan(int64_t rows, int64_t cols, int dtype, int32_t* o
   out[1] = p.maxv;
   out[2] = p.nseg;
   out[3] = (int32_t)p.vps;
+  return kOk;
+}
+
+int tallax_testing_select_edge(int64_t rows, int64_t cols, int dtype, int32_t* out) {
+  if (!out || (dtype != kF32 && dtype != kBF16) || rows < 0 || cols <= 0) {
+    set_error("bad arguments");
+    return kInvalidArgument;
+  }
+  Plan p;
+  const int st = plan_rows(rows, cols, dtype, &p);
+  if (st) return st;
+  const int vec = dtype == kF32 ? 4 : 8;
+  out[0] = p.nt == kNTS && whole_row_edge(nullptr, cols, part_cols_of(cols, p.parts > 1 ? p.parts : 1, vec), 16 / vec);
   return kOk;
 }
 

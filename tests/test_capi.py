@@ -68,6 +68,19 @@ def test_work_split_without_gpu():
         assert p["threads"] == 256 and p["segments"] > 1, (rows, cols, p)
 
 
+def test_work_split_names_the_launched_instance():
+    """EDGE of the reported kernel: true where a row or part is not whole
+    16-byte vectors, parts of rows that do not divide among them."""
+    from tallax_amd import _lib
+    for rows, cols, dt, edge in [(67, 151937, _lib.F32, "true"), (64, 220001, _lib.F32, "true"),
+                                 (64, 155653, _lib.BF16, "true"), (70, 200003, _lib.BF16, "true"),
+                                 (128, 151936, _lib.F32, "false"), (33, 77830, _lib.F32, "true"),
+                                 (256, 128256, _lib.BF16, "false"), (256, 128260, _lib.BF16, "true"),
+                                 (8, 32768, _lib.F32, "false"), (8, 32769, _lib.F32, "true")]:
+        name = _lib.select_plan(rows, cols, dt)["kernel"]
+        assert name.split(" ")[3].startswith(edge), (rows, cols, name)
+
+
 def test_sort_workspace_contract_without_gpu():
     from tallax_amd import _lib
     L = _lib.LIB
