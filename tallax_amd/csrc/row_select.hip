@@ -753,9 +753,9 @@ __device__ __forceinline__ uint32_t min_offset_from_min(const uint4 v) {
 // kernel's hot code (the kernel's code size sets its instruction-cache
 // footprint).
 template <int DT, int V, int NT>
-__device__ __attribute__((noinline)) void fill_ineligible(const uint4* row_base, int nv, int mis, int cols, int n,
-                                                          uint32_t pmin, uint32_t pinf, uint64_t* list, int* red,
-                                                          uint32_t* tmp) {
+__device__ __attribute__((noinline)) void fill_ineligible(const uint4* row_base, int nv, int mis, int cols,
+                                                          int live, int n, uint32_t pmin, uint32_t pinf,
+                                                          uint64_t* list, int* red, uint32_t* tmp) {
   constexpr bool kBF = DT == kBF16;
   constexpr int VEC = ElemT<DT>::VEC, NW = NT / kWave;
   constexpr uint32_t kMinKey = kBF ? 0x0080FFFFu : 0x00800000u;  // global keys of the three classes
@@ -779,7 +779,7 @@ __device__ __attribute__((noinline)) void fill_ineligible(const uint4* row_base,
     pinf |= tmp[NW + i];
   }
   constexpr uint32_t kAll = (1u << V) - 1u;
-  int r = kMaxK - n, base = n;
+  int r = (live < kMaxK ? live : kMaxK) - n, base = n;
 #pragma unroll 1
   for (int c = 0; c < 3 && r > 0; ++c) {  // block-uniform
     uint32_t pres = c == 0 ? pmin : (c == 1 ? pinf : kAll);
@@ -1070,8 +1070,8 @@ void seg_select_kernel(SelArgs a) {
   block_select(sh, (const int*)sh.wc);
   for (int i = tid; i < kRun; i += NT) sh.list64[i] = S::to_global(sh.list[i], seg_e0);
   if (fill_from < kRun) {  // its first barriers order the writes above before its own
-    fill_ineligible<DT, MAXV, NT>(rv.base + s0, (int)(s1 - s0), -(int)seg_e0, (int)a.cols, fill_from, pmin, pinf,
-                                  sh.list64, sh.red, (uint32_t*)stage);
+    fill_ineligible<DT, MAXV, NT>(rv.base + s0, (int)(s1 - s0), -(int)seg_e0, (int)a.cols, live_hi - live_lo,
+                                  fill_from, pmin, pinf, sh.list64, sh.red, (uint32_t*)stage);
   }
   __syncthreads();
   if (a.nseg == 1 && !a.lists_only) {
@@ -1597,7 +1597,7 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   const bool fill = ss.ovf == 0 && n < kq && thr == kFloor;  // block-uniform
   // an overflowing staging region or more than kCandCap candidates: heavy ties
   const bool tie = !fill && (ss.ovf != 0 || n < kq || n > kCandCap);
-  if (fill) fill_ineligible<DT, V, kNTS>(rv.base, nv, rv.mis, cols, n, pmin, pinf, sh.list64, sh.red, &ss.vsi[0][0]);
+  if (fill) fill_ineligible<DT, V, kNTS>(rv.base, nv, rv.mis, cols, cols, n, pmin, pinf, sh.list64, sh.red, &ss.vsi[0][0]);
   if (tie) {
     stream_tie_path<DT, V>(rv.base, nv, rv.mis, cols, sh, stage);
   } else if (n > 0) {

@@ -72,3 +72,23 @@ def test_uneven_parts(gpu, rows, cols, k, dtype, kind, parts):
                                     (64, "sorted_desc"), (128, "special")])
 def test_bound_of_short_rows(gpu, cols, dtype, k, kind):
     _check(gpu, 40, cols, k, dtype, kind, 1024, 1)
+
+
+# a last segment of a handful of elements, fewer than a list holds: nothing
+# ineligible in it, or all of it
+@pytest.mark.parametrize("rows,cols,dtype", [(4, 77827, "f32"), (2, 155653, "f32"), (5, 311299, "f32"),
+                                             (3, 155653, "bf16"), (2, 163841, "bf16")])
+@pytest.mark.parametrize("kind", ["normal", "masked_mix", "special"])
+@pytest.mark.parametrize("tail", [None, np.nan, -np.inf])
+def test_short_last_segment(gpu, rows, cols, dtype, kind, tail):
+    from tallax_amd import _lib, tax
+    print(f"short last segment rows={rows} cols={cols} {dtype} {kind} {tail}", flush=True)
+    x = _make(rows, cols, kind, seed=cols)
+    if tail is not None:
+        x[:, -8:] = tail
+    xd, xv = to_dev(x, dtype, gpu), host_values(x, dtype)
+    assert _lib.select_plan(rows, cols, _lib.dtype_code(xd))["threads"] == 256
+    vals, idx = tax.top_k(xd, 128)
+    ov, oi = O.top_k(xv, 128, dtype)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    assert np.array_equal(bits(from_dev_vals(vals)), bits(ov))
