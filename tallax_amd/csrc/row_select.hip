@@ -538,7 +538,7 @@ __device__ __forceinline__ int32_t vec_omax(const uint4 v) {
 // canonical key lies between a NaN's and -inf's.
 // Returns this wave's number of appended candidates.  Every thread calls it.
 // ---------------------------------------------------------------------------
-template <int DT, int MAXV, int NT, int SG = kStage>
+template <int DT, int MAXV, int NT>
 __device__ __attribute__((noinline)) int tie_select(const uint4* base, int64_t s0, int64_t s1, int lbase,
                                                     int live_lo, int live_hi, uint32_t gbase, int k,
                                                     typename Sel<DT, (NT * MAXV * ElemT<DT>::VEC > 65535)>::Comp* reg,
@@ -647,15 +647,15 @@ __device__ __attribute__((noinline)) int tie_select(const uint4* base, int64_t s
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
-    for (int c = 0; c < (MAXV + SG - 1) / SG; ++c) {
+    for (int c = 0; c < (MAXV + kStage - 1) / kStage; ++c) {
       if (pass == 1 && rest <= 0) break;
 #pragma unroll
-      for (int u = 0; u < SG; ++u)
-        if (c * SG + u < MAXV) stage[u * NT + tid] = raw[c * SG + u];
+      for (int u = 0; u < kStage; ++u)
+        if (c * kStage + u < MAXV) stage[u * NT + tid] = raw[c * kStage + u];
 #pragma unroll 1
-      for (int u = 0; u < SG && c * SG + u < MAXV; ++u) {
+      for (int u = 0; u < kStage && c * kStage + u < MAXV; ++u) {
         if (pass == 1 && rest <= 0) break;
-        const int li0 = lbase + (c * SG + u) * NT * VEC;
+        const int li0 = lbase + (c * kStage + u) * NT * VEC;
         const uint4 vv = stage[u * NT + tid];
         const uint32_t lm = live_bits(li0);
         uint32_t mask = 0;
@@ -1219,18 +1219,17 @@ __global__ __launch_bounds__(kWave) void seg_merge64_pair_kernel(SelArgs a) {
 //      bucket.  The first 128 (64) ranks are the row's top-128 (64) in order.
 // Rows with fewer than 128 eligible elements rank them and take the rest of
 // the list by class (fill_ineligible).  Rows whose staged vectors or
-// candidates overflow (heavy ties: constant rows, long tie blocks) take
-// tie_select over the whole row instead (stream_tie_path).  Both rare paths
+// candidates overflow (heavy ties: constant rows, long tie blocks) raise the
+// bound to the k-th largest key first (raise_staged, raise_row).  The rare paths
 // are out of line: the kernel's hot code is 31 KB instead of 50 KB (measured
 // at config 4 together with step 3's per-vector staging: 16.2 -> 15.8 us).
 // ---------------------------------------------------------------------------
 constexpr int kNTS = 1024;
-constexpr int kStageCap = 128;   // staged vectors per wave
+constexpr int kStageCap = 256;   // staged vectors per wave
 constexpr int kCandCap = 1024;   // candidates (one per thread in the ranking)
 constexpr int kBuckets = 1024;
 
 struct StreamShared {
-  uint4 vst[kNTS / kWave][kStageCap];      // staged vectors, per wave     32 KiB
   uint32_t vsi[kNTS / kWave][kStageCap];   // their first element's row index
   uint64_t cand[kCandCap + 8];             // candidates, then in bucket order (+8: unguarded reads)
   int hist[kBuckets];                      // bucket counts, then bucket starts
@@ -1239,6 +1238,15 @@ struct StreamShared {
   uint32_t posted;  // bit w: wave w (< 8) has its bound term in wl
   int ncand;
   int ovf;                                 // a wave's staged vectors overflowed its region
+  uint64_t list64[kRun];
+  float samp_g[kRun];                      // sampler: Gumbel noise of the top-128
+  int red[kNTS / kWave];
+  // raise_threshold: a probe's count, smallest and largest t per wave, two probes in turn
+  int tie_c[2][kNTS / kWave];
+  uint32_t tie_mn[2][kNTS / kWave], tie_mx[2][kNTS / kWave];
+  int tie_last;                            // the last range of vectors that is needed
+  uint32_t tie_k, tie_top;                 // the new threshold, the row's largest key
+  uint4 vst[kNTS / kWave][kStageCap];      // staged vectors, per wave: 64 KiB, past the offsets of the rest
 };
 
 // lanes below this one in the wave
@@ -1308,52 +1316,251 @@ __device__ __forceinline__ uint32_t pass_mask_ge(const uint4 vv, uint32_t thr) {
   return m;
 }
 
-// Rows whose staged vectors or candidates overflow (heavy ties): tie_select
-// over the whole row, then the block's merge, into the sorted 128-entry list.
-// Out of line, like fill_ineligible.
-template <int DT, int V>
-__device__ __attribute__((noinline)) void stream_tie_path(
-    const uint4* base, int nv, int mis, int cols,
-    SegShared<typename Sel<DT, (kNTS * V * ElemT<DT>::VEC > 65535)>::Comp, kNTS>& sh, uint4* stage) {
-  using ST = Sel<DT, (kNTS * V * ElemT<DT>::VEC > 65535)>;
-  constexpr int VEC = ElemT<DT>::VEC;
+// ---------------------------------------------------------------------------
+// Rows with more candidates than the rank takes (heavy ties): the threshold is
+// raised to the k-th largest key K and the candidates are found again: the
+// elements above K and, where those equal to K are many, the ones in the first
+// vectors of the row that hold enough of them (at most 128 + 256 in all).
+//   K lies in [thr, +inf], and at least k elements are >= thr (where fewer are,
+// thr being the eligibility floor, all of them are candidates).  A probe in the
+// middle of the range counts the elements at or above it, and finds the
+// smallest of them and the largest below: the new end of the range, so the
+// range ends on keys that occur and a row of few distinct values takes three to
+// five probes.  (A bisection over all key bits, counting from registers, took 17
+// or 33, then an exact selection element by element: bf16 [4, 151936] of ten
+// values 139 -> 22 us, f32 [100, 65536] 87 -> 27, parts of [33, 100003] 76 -> 21,
+// [64, 155653] 78 -> 29.)  Bound by VALU issue: 4 instructions per
+// f32 element and probe, 7 per pair of bf16 ones.
+//   raw keys are compared (tie_select describes them): with t = raw - raw_thr(mid)
+// modulo the key width, the elements from mid to +inf are t <= +inf - mid, the
+// smallest of them has the smallest t and the largest one below mid the
+// largest (a NaN has neither).
+// The thread's elements: raw[j], vector number vec_no(j) of the row.
+// ---------------------------------------------------------------------------
+template <int DT, int NV, typename VecNo>
+__device__ __forceinline__ void raise_threshold(uint4 (&raw)[NV], VecNo vec_no, int nv, int mis, uint32_t thr, int k,
+                                                StreamShared& ss) {
+  constexpr bool kBF = DT == kBF16;
+  constexpr int VEC = ElemT<DT>::VEC, NW = kNTS / kWave;
+  using S = Sel<DT, true>;
+  constexpr uint32_t kZeroKey = kBF ? 0x8000u : 0x80000000u;
+  constexpr uint32_t kInfKey = kBF ? 0xFF80u : 0xFF800000u;
+  constexpr uint32_t kMask = kBF ? 0xFFFFu : 0xFFFFFFFFu;
   const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
-  const int lbase = tid * VEC;
-  const int64_t seg_e0 = -(int64_t)mis;
-  const int live_lo = mis;
-  const int live_hi = cols + mis < nv * VEC ? cols + mis : nv * VEC;
-  const int wcnt = tie_select<DT, V, kNTS, 2>(base, 0, nv, lbase, live_lo, live_hi, (uint32_t)seg_e0, kMaxK,
-                                              sh.cand + w * Geo<kNTS>::WCAP, sh.red, stage);
-  if (l == 0) sh.wc[w] = wcnt;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    uint32_t d[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = kBF ? raw_key2_bf16(d[i]) : raw_key_f32(d[i]);
+    raw[j] = make_uint4(d[0], d[1], d[2], d[3]);
+  }
+  uint32_t lo = thr, hi = kInfKey + 1u;  // count(>= lo) >= k > count(>= hi)
+  uint32_t top = 0;                      // the row's largest key
+  int c_lo = 0x7FFFFFFF, c_hi = 0;       // those counts (c_lo: unknown at first)
+  uint32_t mid = hi;                     // the first probe finds the largest key
+#pragma unroll 1
+  for (int it = 0;; it ^= 1) {
+    const uint32_t mr = S::raw_thr(mid), span = kInfKey - mr;  // mid = +inf + 1: no element passes
+    int c = 0;
+    uint32_t tmin, tmax;
+    if constexpr (kBF) {
+      const ushort2_t m2 = __builtin_bit_cast(ushort2_t, mr * 0x10001u);
+      const ushort2_t s2 = __builtin_bit_cast(ushort2_t, (mid > kInfKey ? 0u : span) * 0x10001u);
+      const ushort2_t one = __builtin_bit_cast(ushort2_t, 0x00010001u);
+      ushort2_t out = __builtin_bit_cast(ushort2_t, 0u), mn = __builtin_bit_cast(ushort2_t, ~0u), mx = out;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const ushort2_t t = __builtin_bit_cast(ushort2_t, dword_of(raw[j], i)) - m2;
+          out += __builtin_elementwise_min(__builtin_elementwise_sub_sat(t, s2), one);
+          mn = __builtin_elementwise_min(mn, t);
+          mx = __builtin_elementwise_max(mx, t);
+        }
+      }
+      c = NV * VEC - (int)out[0] - (int)out[1];
+      tmin = mn[0] < mn[1] ? mn[0] : mn[1];
+      tmax = mx[0] > mx[1] ? mx[0] : mx[1];
+    } else {
+      tmin = ~0u;
+      tmax = 0u;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t t = dword_of(raw[j], i) - mr;
+          c += t <= span ? 1 : 0;
+          tmin = t < tmin ? t : tmin;
+          tmax = t > tmax ? t : tmax;
+        }
+      }
+    }
+    if (mid > kInfKey) c = 0;
+    c = wave_sum_i(c);
+    tmin = wave_min_u32(tmin);
+    tmax = wave_max_u32(tmax);
+    if (l == 0) {
+      ss.tie_c[it][w] = c;
+      ss.tie_mn[it][w] = tmin;
+      ss.tie_mx[it][w] = tmax;
+    }
+    __syncthreads();  // the other buffer is read before this barrier and written after it
+    c = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      c += ss.tie_c[it][i];
+      tmin = ss.tie_mn[it][i] < tmin ? ss.tie_mn[it][i] : tmin;
+      tmax = ss.tie_mx[it][i] > tmax ? ss.tie_mx[it][i] : tmax;
+    }
+    // canonical keys of the smallest at or above mid, the largest below it
+    const uint32_t up = (mr + tmin) & kMask, dn = (mr + tmax) & kMask;
+    if (c >= k) {
+      lo = up == kZeroKey - 1u ? kZeroKey : (up > mid ? up : mid);
+      c_lo = c;
+      if (c == k) break;
+    } else {
+      const uint32_t d = dn == kZeroKey - 1u ? kZeroKey : dn;
+      if (mid > kInfKey) top = d;
+      hi = d < mid ? d + 1u : mid;
+      c_hi = c;
+    }
+    if (hi <= lo + 1u) break;  // K = lo
+    mid = lo + (hi - lo) / 2u;
+  }
+  // Elements equal to K: all of them, or those in the row's first vectors, in
+  // ranges of 2^sh vectors, that hold the k - c_hi first ones.
+  const uint32_t kr = S::raw_thr(lo), kspan = kInfKey - kr;
+  int sh = 0;
+  while (((nv - 1) >> sh) >= kBuckets) ++sh;
+  uint32_t vlast = ~0u;
+  auto eq_mask = [&](const uint4 x) -> uint32_t {  // elements equal to K (raw keys; +-0 are one)
+    uint32_t m = 0;
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) {
+      const uint32_t r = elem_bits<DT>(x, q);
+      m |= (r == kr || r == lo ? 1u : 0u) << q;
+    }
+    return m;
+  };
+  if (c_lo > k + 64) {  // block-uniform
+    for (int i = tid; i < kBuckets; i += kNTS) ss.hist[i] = 0;
+    if (tid == 0) ss.tie_last = kBuckets - 1;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const uint32_t m = eq_mask(raw[j]);
+      if (m) atomicAdd(&ss.hist[vec_no(j) >> sh], (int)__popc(m));
+    }
+    __syncthreads();
+    if (w == 0) {  // the range that holds the last one needed, 16 ranges per lane
+      constexpr int PER = kBuckets / kWave;
+      int cnt[PER], loc = 0;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        cnt[i] = ss.hist[l * PER + i];
+        loc += cnt[i];
+      }
+      int tot;
+      int run = wave_exscan_i32(loc, tot);
+      const int need = k - c_hi;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        if (run < need && need <= run + cnt[i]) ss.tie_last = l * PER + i;
+        run += cnt[i];
+      }
+    }
+    __syncthreads();
+    vlast = ((uint32_t)ss.tie_last << sh) + ((1u << sh) - 1u);
+  }
+  for (int i = tid; i < kBuckets; i += kNTS) ss.hist[i] = 0;  // the rank's buckets
+  if (tid == 0) {
+    ss.ncand = 0;
+    ss.tie_k = lo;
+    ss.tie_top = top;
+  }
   __syncthreads();
-  block_select(sh, (const int*)sh.wc);
-  for (int i = tid; i < kRun; i += kNTS) sh.list64[i] = ST::to_global(sh.list[i], seg_e0);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const uint4 x = raw[j];
+    const uint32_t v = vec_no(j), e0 = v * VEC - (uint32_t)mis;
+    uint32_t pm = 0;
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) pm |= (elem_bits<DT>(x, q) - kr <= kspan ? 1u : 0u) << q;
+    if (v > vlast) pm &= ~eq_mask(x);
+    if (!__ballot(pm != 0u)) continue;  // wave-uniform
+    int tot;
+    const int pre = wave_exscan_i32(__popc(pm), tot);
+    int b0 = 0;
+    if (l == 0) b0 = atomicAdd(&ss.ncand, tot);
+    int oc = __builtin_amdgcn_readfirstlane(b0) + pre;
+    while (pm) {
+      const int q = __builtin_ctz(pm);
+      pm &= pm - 1u;
+      const uint32_t r = elem_bits<DT>(x, q);
+      if (oc < kCandCap) ss.cand[oc] = make_comp(r == kZeroKey - 1u ? kZeroKey : r, e0 + (uint32_t)q);
+      ++oc;
+    }
+  }
+  __syncthreads();
 }
 
-template <int DT, int V, bool SAMPLE, bool EDGE>
+// More than kCandCap candidates: the threshold is raised over the staged vectors,
+// which hold every one of them.
+template <int DT>
+__device__ __attribute__((noinline)) void raise_staged(int nv, int mis, int wcnt, uint32_t thr, int k,
+                                                       StreamShared& ss) {
+  constexpr int VEC = ElemT<DT>::VEC, NV = kStageCap / kWave;
+  const int w = threadIdx.x / kWave, l = lane_id();
+  uint4 raw[NV];
+  uint32_t vn[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int o = j * kWave + l;
+    raw[j] = o < wcnt ? ss.vst[w][o] : make_uint4(~0u, ~0u, ~0u, ~0u);
+    vn[j] = o < wcnt ? (ss.vsi[w][o] + (uint32_t)mis) / (uint32_t)VEC : 0u;
+  }
+  raise_threshold<DT, NV>(raw, [&](int j) { return vn[j]; }, nv, mis, thr, k, ss);
+}
+
+// A wave had more vectors to stage than its region holds: the row is read again.
+template <int DT, int V>
+__device__ __attribute__((noinline)) void raise_row(const uint4* base, int nv, int mis, int cols, uint32_t thr, int k,
+                                                    StreamShared& ss) {
+  constexpr int VEC = ElemT<DT>::VEC;
+  const int tid = threadIdx.x;
+  uint4 raw[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const int v = j * kNTS + tid;
+    raw[j] = v < nv ? base[v] : make_uint4(~0u, ~0u, ~0u, ~0u);
+  }
+#pragma unroll
+  for (int j = 0; j < V; ++j) {  // slots outside the row become all-ones
+    const int e0 = (j * kNTS + tid) * VEC - mis;
+    if (e0 < 0 || e0 + VEC > cols) raw[j] = kill_slots<DT>(raw[j], e0 < 0 ? -e0 : 0, cols - e0);
+  }
+  raise_threshold<DT, V>(raw, [&](int j) { return (uint32_t)(j * kNTS + tid); }, nv, mis, thr, k, ss);
+}
+
+template <int DT, int V, bool SAMPLE, bool EDGE, bool PARTS = false>
 __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
+  static_assert(!SAMPLE || !PARTS, "parts end in lists");
   using T = ElemT<DT>;
   constexpr int VEC = T::VEC, ES = T::ES, NW = kNTS / kWave;
   static_assert(V <= 31, "one bit per vector in 32-bit masks");
   constexpr bool kBF = DT == kBF16;
   constexpr int KB = kBF ? 16 : 32;  // canonical key bits
-  using ST = Sel<DT, (kNTS * V * VEC > 65535)>;  // the tie path's composites (tie_select's choice)
-  using CT = typename ST::Comp;
   constexpr uint32_t kZeroKey = kBF ? 0x8000u : 0x80000000u;
   constexpr int32_t kPosInf = kBF ? 0x7F80 : 0x7F800000;
   constexpr int32_t kOrdNegInf = kBF ? -32641 : (int32_t)0x807FFFFFu;
   constexpr uint32_t kFloor = kBF ? 0x0081u : 0x00800001u;  // smallest eligible canonical key
   __shared__ StreamShared ss;
-  __shared__ SegShared<CT, kNTS> sh;  // tie path, output list
-  __shared__ uint4 stage[2 * kNTS];   // tie path
   const int tid = threadIdx.x, w = tid / kWave, l = lane_id();
-  // row parts (SAMPLE = false only): workgroup (part, row) of a two-dimensional
-  // grid, so that a row's parts run side by side; its last part may be shorter
-  const bool parts = !SAMPLE && a.part_cols < a.cols;
-  const int64_t row = parts ? blockIdx.y : blockIdx.x;
-  const unsigned part = parts ? blockIdx.x : 0u;
-  const int64_t c0 = (int64_t)((uint64_t)part * (uint32_t)a.part_cols);
-  const int left = (int)(a.cols - c0), cols = SAMPLE || left < a.part_cols ? left : a.part_cols;
+  // PARTS: workgroup (part, row) of a two-dimensional grid, so that a row's
+  // parts run side by side; its last part may be shorter
+  const int64_t row = PARTS ? blockIdx.y : blockIdx.x;
+  const int64_t c0 = PARTS ? (int64_t)((uint64_t)blockIdx.x * (uint32_t)a.part_cols) : 0;
+  const int left = (int)(a.cols - c0), cols = !PARTS || left < a.part_cols ? left : a.part_cols;
   const char* rowp = (const char*)a.x + (size_t)(row * a.cols + c0) * ES;
   const RowVec<ES> rv(rowp);
   const int nv = (cols + rv.mis + VEC - 1) / VEC;  // 1 <= nv <= kNTS * V (host plan)
@@ -1475,7 +1682,7 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
     }
   };
 
-  uint32_t thr, M;
+  uint32_t thr;
   uint32_t pmin = 0, pinf = 0;  // rows with thr at the floor: the vectors that may hold finfo.min / -inf
   // ---- 2. the bound L from waves 0..7 alone: the minimum over them of each
   // one's 16th largest thread maximum, so at least 128 elements of the row
@@ -1588,19 +1795,25 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
   __syncthreads();
   // M: at least the largest candidate key (waves 0..7 post their largest
   // element, waves 8..15 their largest candidate), all the rank needs
-  M = ss.wm[0];
+  uint32_t M = ss.wm[0];
 #pragma unroll
   for (int i = 1; i < NW; ++i) M = ss.wm[i] > M ? ss.wm[i] : M;
-  const int n = ss.ncand;
+  int n = ss.ncand;
   // fewer than 128 with thr at the eligibility floor: every eligible element
   // of the row is a candidate, the rest of the list is ineligible elements
-  const bool fill = ss.ovf == 0 && n < kq && thr == kFloor;  // block-uniform
+  // (and so where vectors of positive NaNs overflow the staging regions)
+  const bool floor = thr == kFloor;  // block-uniform
   // an overflowing staging region or more than kCandCap candidates: heavy ties
-  const bool tie = !fill && (ss.ovf != 0 || n < kq || n > kCandCap);
-  if (fill) fill_ineligible<DT, V, kNTS>(rv.base, nv, rv.mis, cols, cols, n, pmin, pinf, sh.list64, sh.red, &ss.vsi[0][0]);
-  if (tie) {
-    stream_tie_path<DT, V>(rv.base, nv, rv.mis, cols, sh, stage);
-  } else if (n > 0) {
+  if (ss.ovf != 0 || n > kCandCap) {  // block-uniform
+    if (ss.ovf != 0) raise_row<DT, V>(rv.base, nv, rv.mis, cols, thr, kq, ss);
+    else raise_staged<DT>(nv, rv.mis, wcnt, thr, kq, ss);
+    thr = ss.tie_k;
+    M = ss.tie_top;
+    n = ss.ncand;
+  }
+  if (floor && n < kq)
+    fill_ineligible<DT, V, kNTS>(rv.base, nv, rv.mis, cols, cols, n, pmin, pinf, ss.list64, ss.red, &ss.vsi[0][0]);
+  if (n > 0) {
     // ---- 4. bucket rank
     const uint32_t range = M - thr;  // the candidates' keys lie in [thr, M]
     int shift = 0;
@@ -1651,17 +1864,17 @@ __global__ __launch_bounds__(kNTS) void stream_select_kernel(SelArgs a) {
         const uint32_t k = comp_key(c);
         uint32_t key = k;
         if (kBF) key = k >= 0x8000u ? (k << 16) : ((k << 16) | 0xFFFFu);
-        sh.list64[r] = make_comp(key, ~(uint32_t)c);
+        ss.list64[r] = make_comp(key, ~(uint32_t)c);
       }
     }
   }
   __syncthreads();
-  if (!a.lists_only) {
-    finalize_row<DT, SAMPLE>(a, row, sh.list64, sh.samp_g, rp);
+  if (!PARTS && !a.lists_only) {
+    finalize_row<DT, SAMPLE>(a, row, ss.list64, ss.samp_g, rp);
   } else {
-    uint64_t* dst = a.ws_lists + (size_t)(parts ? row * gridDim.x + part : row) * kRun;
+    uint64_t* dst = a.ws_lists + (size_t)(PARTS ? row * gridDim.x + blockIdx.x : row) * kRun;
     const uint64_t off = (uint64_t)(a.col_offset + c0);
-    for (int i = tid; i < kq; i += kNTS) dst[i] = sh.list64[i] ? sh.list64[i] - off : 0ull;
+    for (int i = tid; i < kq; i += kNTS) dst[i] = ss.list64[i] ? ss.list64[i] - off : 0ull;
   }
 }
 
@@ -1858,7 +2071,6 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
   // parts: the whole-row kernel writes each part's list (no sampling), the
   // merge kernel finishes the row
   SelArgs h = a0;
-  h.part_cols = (int)a0.cols;
   // top-k with k <= 64 reads the first 64 places of a row's (or a part's) list
   if (!SAMPLE && !a0.lists_only && a0.k <= kWave) h.list_k = kWave;
   if (p.parts > 1) {
@@ -1871,11 +2083,11 @@ static int launch_select(const SelArgs& a0, const Plan& p, hipStream_t s, const 
     const bool edge = whole_row_edge(a.x, a.cols, a.part_cols, ElemT<DT>::ES);
     const dim3 g((unsigned)p.parts, (unsigned)a.rows), b(kNTS);
     if (p.maxv == 19) {
-      if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true>), g, b, 0, s, a);
-      else hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, false>), g, b, 0, s, a);
+      if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, true, true>), g, b, 0, s, a);
+      else hipLaunchKernelGGL((stream_select_kernel<DT, 19, false, false, true>), g, b, 0, s, a);
     } else {
-      if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 16, false, true>), g, b, 0, s, a);
-      else hipLaunchKernelGGL((stream_select_kernel<DT, 16, false, false>), g, b, 0, s, a);
+      if (edge) hipLaunchKernelGGL((stream_select_kernel<DT, 16, false, true, true>), g, b, 0, s, a);
+      else hipLaunchKernelGGL((stream_select_kernel<DT, 16, false, false, true>), g, b, 0, s, a);
     }
   } else if (p.nt == kNTS) {
     const bool edge = whole_row_edge(a.x, a.cols, a.cols, ElemT<DT>::ES);

@@ -92,3 +92,57 @@ def test_short_last_segment(gpu, rows, cols, dtype, kind, tail):
     ov, oi = O.top_k(xv, 128, dtype)
     assert np.array_equal(idx.cpu().numpy(), oi)
     assert np.array_equal(bits(from_dev_vals(vals)), bits(ov))
+
+
+# whole rows and parts with too many candidates: many elements equal to the
+# k-th largest, in the first vectors of the row, in its last ones, everywhere;
+# few and many distinct values; candidates staged and not; both zeros; NaNs
+def _tied(rows, cols, kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "rounded":
+        return np.round(rng.standard_normal((rows, cols)) * 1.5).astype(np.float32)
+    if kind == "dense":       # a tenth of the row at the top value
+        return (rng.random((rows, cols)) < 0.1).astype(np.float32) + 3
+    if kind == "late":        # the ties in the row's last vectors, a few larger ones anywhere
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        x[:, -min(cols, 2500):] = 7.0
+        for r in range(rows):
+            x[r, rng.choice(cols, min(cols, 40), replace=False)] = 8.0 + rng.integers(0, 3)
+        return x
+    if kind == "zeros":       # the k-th largest is a zero of either sign, NaNs and infinities about
+        x = -np.abs(rng.standard_normal((rows, cols))).astype(np.float32)
+        x[rng.random((rows, cols)) < 0.2] = 0.0
+        x[rng.random((rows, cols)) < 0.2] = -0.0
+        x[rng.random((rows, cols)) < 0.1] = np.nan
+        x[:, ::997] = np.inf
+        return x
+    if kind == "nans":        # vectors of positive NaNs, few or no eligible values
+        x = np.full((rows, cols), np.nan, np.float32)
+        for r in range(rows - 1):
+            x[r, rng.choice(cols, 60, replace=False)] = rng.integers(-2, 3, 60)
+            x[r, rng.choice(cols, 10, replace=False)] = -np.inf
+        return x
+    if kind == "ramp":        # no ties, yet one thread's vectors hold the largest
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        x[:, :min(cols, 4000)] += 50 + np.arange(min(cols, 4000), dtype=np.float32) / 64
+        return x
+    x = np.full((rows, cols), -5.0, np.float32)   # negative constant
+    x[:, cols // 2] = np.finfo(np.float32).min
+    return x
+
+
+@pytest.mark.parametrize("kind", ["rounded", "dense", "late", "zeros", "nans", "ramp", "negconst"])
+@pytest.mark.parametrize("cols,dtype", [(1100, "f32"), (8193, "f32"), (40000, "f32"), (77820, "f32"), (151936, "f32"),
+                                        (4097, "bf16"), (25000, "bf16"), (65537, "bf16"), (128256, "bf16"),
+                                        (155641, "bf16"), (262144, "bf16")])
+@pytest.mark.parametrize("k", [50, 128])
+def test_raised_threshold(gpu, cols, dtype, kind, k):
+    from tallax_amd import _lib, tax
+    print(f"raised threshold cols={cols} k={k} {dtype} {kind}", flush=True)
+    x = _tied(4, cols, kind, seed=cols + k)
+    xd, xv = to_dev(x, dtype, gpu), host_values(x, dtype)
+    assert _lib.select_plan(4, cols, _lib.dtype_code(xd))["threads"] == 1024
+    vals, idx = tax.top_k(xd, k)
+    ov, oi = O.top_k(xv, k, dtype)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    assert np.array_equal(bits(from_dev_vals(vals)), bits(ov))
