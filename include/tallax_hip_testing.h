@@ -38,10 +38,11 @@ int tallax_testing_lane_ops(uint32_t* out, tallax_stream_t stream);
  * out[3] vectors per segment.  Host only: no device work. */
 int tallax_testing_select_plan(int64_t rows, int64_t cols, int dtype, int32_t* out);
 
-/* out[0] = 1 where those entry points launch the whole-row kernel's instance
- * for rows or parts that are not whole aligned 16-byte vectors (a 16-byte
- * aligned base assumed), else 0.  Host only: no device work. */
-int tallax_testing_select_edge(int64_t rows, int64_t cols, int dtype, int32_t* out);
+/* The same four words for top-k with k <= 64 (`few` != 0), or for k > 64 and
+ * the sampler (0, tallax_testing_select_plan's), and out[4] = 1 where the
+ * whole-row kernel's instance for rows or parts that are not whole aligned
+ * 16-byte vectors is launched (a 16-byte aligned base assumed), else 0. */
+int tallax_testing_select_route(int64_t rows, int64_t cols, int dtype, int few, int32_t* out);
 
 /* tallax_top_dynamic_k with its path chosen by `path`: 0 (what
  * tallax_top_dynamic_k runs) settles rows from the exact kernel's per-segment

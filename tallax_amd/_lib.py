@@ -64,7 +64,7 @@ _SIGNATURES = {
     "tallax_testing_read_bytes": ([_c_p, _c_i64, _c_int, _c_p, _c_p], _c_int),
     "tallax_testing_lds_atomic_order": ([_c_p, _c_i64, _c_int, _c_p, _c_p], _c_int),
     "tallax_testing_select_plan": ([_c_i64, _c_i64, _c_int, _c_p], _c_int),
-    "tallax_testing_select_edge": ([_c_i64, _c_i64, _c_int, _c_p], _c_int),
+    "tallax_testing_select_route": ([_c_i64, _c_i64, _c_int, _c_int, _c_p], _c_int),
     "tallax_testing_top_dynamic_k_path": ([_c_p, _c_int, _c_i64, _c_i64, _c_p, _c_int, _c_int, _c_int, _c_p, _c_int,
                                            _c_int, _c_int, _c_d, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_sz, _c_p, _c_int],
                                           _c_int),
@@ -187,16 +187,15 @@ def select_plan(rows: int, cols: int, dtype: int, k: int = 128, sample: bool = T
     Rows of several segments or parts finish in seg_merge64_pair_kernel (two
     lists) or seg_merge64_kernel for top-k with k <= 64 (no sampler), else in
     seg_merge_kernel."""
-    out = (ctypes.c_int32 * 4)()
-    check(LIB.tallax_testing_select_plan(rows, cols, dtype, out), "select_plan")
-    nt, maxv, nseg, vps = list(out)
+    out = (ctypes.c_int32 * 5)()
+    few = not sample and k <= 64
+    check(LIB.tallax_testing_select_route(rows, cols, dtype, int(few), out), "select_plan")
+    nt, maxv, nseg, vps, edge = list(out)
     dt = {F32: 0, BF16: 1}[dtype]
-    merge = ("seg_merge64_pair_kernel" if nseg <= 2 else "seg_merge64_kernel") if (not sample and k <= 64) \
-        else "seg_merge_kernel"
+    merge = ("seg_merge64_pair_kernel" if nseg <= 2 else "seg_merge64_kernel") if few else "seg_merge_kernel"
     if nt == 1024:
         # EDGE: rows (or parts) not a whole number of 16-byte vectors (a 16-byte aligned base assumed)
-        check(LIB.tallax_testing_select_edge(rows, cols, dtype, out), "select_plan")
-        edge = "true" if out[0] else "false"
+        edge = "true" if edge else "false"
         if nseg == 1:
             name = f"stream_select_kernel<{dt}, {maxv}, SAMPLE, {edge}>"
         else:

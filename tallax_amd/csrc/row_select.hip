@@ -65,6 +65,9 @@ constexpr int kTargetBlocks = 1024;        // ~4 workgroups per CU on 256 CUs
 constexpr int kPartsMaxBlocks = 512;       // whole-row parts: two rounds of one workgroup per CU at most
 constexpr int kUnevenMinBlocks = 128;      // parts of a row that does not divide: one round that fills
 constexpr int kUnevenMaxBlocks = 256;      // at least half of the CUs (plan_rows)
+constexpr int kUnevenMinVecFew = 8192;     // shortest such part, in 16-byte vectors: top-k with k <= 64,
+constexpr int kUnevenMinVecBf16 = 6144;    // other bf16 calls
+constexpr int kUnevenMinRowsFew = 64;      // fewest such rows: bf16 top-k with k <= 64
 
 struct SelArgs {
   const void* x;
@@ -1942,40 +1945,6 @@ struct Plan {
   int parts;  // > 1: whole-row kernel on that many parts of each row, then the merge
 };
 
-// Work split.  A row of nv 16-byte vectors is handled either
-//   * whole by one 1024-thread workgroup of stream_select_kernel (up to 19
-//     vectors per thread) whenever the row fits: no merge kernel at all.  At
-//     small row counts one workgroup per row leaves most CUs idle, but a
-//     256 KiB row streams into one workgroup in ~6 us (at most ~40 GB/s),
-//     less than the segment path's bound-after-loads plus second launch
-//     (measured, A/B: sampler [1, 128256] bf16 13.0 -> 9.0 us, [64, 128256]
-//     16.6 -> 11.7; top-k [8, 32768] f32 9.90 -> 8.05, [100, 65472] f32
-//     16.7 -> 11.8; 19 vectors per thread for the 151936-wide bf16
-//     vocabulary: sampler [64, 151936] 20.5 -> 12.7, [256, 151936] 25.2 ->
-//     17.8; no shape slower); or
-//   * as 2-4 parts of at most 19 vectors per thread when the row
-//     divides and rows x parts <= kPartsMaxBlocks: the whole-row kernel
-//     writes each part's top-128 list (rows of the [parts x rows, cols /
-//     parts] view, column offsets added back), then the per-row merge
-//     (config 3, [128, 151936] f32: 21.50 -> 20.05 us; f32 sampler
-//     [64, 128256] 19.5 -> 15.7, [64, 201088] 26.9 -> 17.2; at more blocks
-//     the segments win: [256, 201088] 46.5 against 50.4, [512, 151936]
-//     top-k 55.1 against 62.6); rows that do not divide take parts of whole
-//     vectors, the last one shorter, where 128 to 256 part workgroups make
-//     one round over at least half of the CUs (f32, segments -> parts: sampler
-//     [64, 151937] 24.3 -> 19.3 us, [128, 151937] 26.7 -> 23.1, [64, 220001]
-//     28.8 -> 21.0; top-k k = 50 [64, 151937] 18.3 -> 17.0; bf16 sampler
-//     [48, 220001] 22.9 -> 17.8, [128, 220001] masked 33.0 -> 26.1).  Fewer rows
-//     do better in segments, which spread each row over more CUs (top-k
-//     [16, 151937] 12.2 against 15.6 us, masked sampler [32, 220001] 21.2
-//     against 23.3), and so does a second round ([128, 220001] f32 sampler
-//     34.0 against 36.0); or
-//   * in segments of 256 x MAXV vectors, MAXV in {4, 8, 16, 19}: the largest that
-//     still gives ~4 workgroups per CU over the launch, then a per-row merge;
-//     where 16 gives more than one residency round (4 workgroups per CU,
-//     kTargetBlocks) and 19 gives exactly one, MAXV = 19 (config 3: 8
-//     segments of 19 vectors per thread instead of 10 of 16, measured
-//     22.03 -> 21.45 us).
 // Columns per part: equal parts when the row divides, else whole vectors with a
 // shorter last part.
 static int64_t part_cols_of(int64_t cols, int np, int vec) {
@@ -1991,7 +1960,47 @@ static bool whole_row_edge(const void* x, int64_t cols, int64_t part_cols, int e
   return ((uintptr_t)x % 16) != 0 || (cols * es) % 16 != 0 || (part_cols * es) % 16 != 0;
 }
 
-static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
+// Work split.  A row of nv 16-byte vectors is handled either
+//   * whole by one 1024-thread workgroup of stream_select_kernel (up to 19
+//     vectors per thread) whenever the row fits: no merge kernel at all.  At
+//     small row counts one workgroup per row leaves most CUs idle, but a
+//     256 KiB row streams into one workgroup in ~6 us (at most ~40 GB/s),
+//     less than the segment path's bound-after-loads plus second launch
+//     (measured, A/B: sampler [1, 128256] bf16 13.0 -> 9.0 us, [64, 128256]
+//     16.6 -> 11.7; top-k [8, 32768] f32 9.90 -> 8.05, [100, 65472] f32
+//     16.7 -> 11.8; 19 vectors per thread for the 151936-wide bf16
+//     vocabulary: sampler [64, 151936] 20.5 -> 12.7, [256, 151936] 25.2 ->
+//     17.8; no shape slower); or
+//   * as 2-4 parts of at most 19 vectors per thread when the row
+//     divides and rows x parts <= kPartsMaxBlocks: the whole-row kernel
+//     writes each part's top-128 list, then the per-row merge
+//     (config 3, [128, 151936] f32: 21.50 -> 20.05 us; f32 sampler
+//     [64, 128256] 19.5 -> 15.7, [64, 201088] 26.9 -> 17.2; at more blocks
+//     the segments win: [256, 201088] 46.5 against 50.4, [512, 151936]
+//     top-k 55.1 against 62.6); rows that do not divide take parts of whole
+//     vectors, the last one shorter, where 128 to 256 part workgroups make
+//     one round over at least half of the CUs (f32, segments -> parts: sampler
+//     [64, 151937] 24.3 -> 19.3 us, [128, 151937] 26.7 -> 23.1, [64, 220001]
+//     28.8 -> 21.0; top-k k = 50 [64, 151937] 18.3 -> 17.0; bf16 sampler
+//     [48, 220001] 22.9 -> 17.8, [128, 220001] masked 33.0 -> 26.1).  Fewer rows
+//     do better in segments, which spread each row over more CUs (top-k
+//     [16, 151937] 12.2 against 15.6 us, masked sampler [32, 220001] 21.2
+//     against 23.3), and so does a second round ([128, 220001] f32 sampler
+//     34.0 against 36.0).  Lists of 64 places (`few`: top-k, k <= 64) are shorter work
+//     in segments: there two or three parts of at least kUnevenMinVecFew vectors,
+//     and bf16 rows from kUnevenMinRowsFew on (k = 50, segments / parts: f32
+//     [32, 77827] 11.2 / 12.1 us, [43, 100003] 15.3 / 13.0, [64, 77827] 15.4 / 12.6;
+//     bf16 [32, 200003] 12.3 / 14.4, [43, 311299] 14.2 / 16.1, [64, 311299]
+//     18.5 / 17.6, [43, 155653] 12.4 / 15.0).  Other bf16 calls take parts of at
+//     least kUnevenMinVecBf16 (sampler [32, 155653] 15.7 / 16.6, [32, 200003]
+//     18.0 / 16.7); or
+//   * in segments of 256 x MAXV vectors, MAXV in {4, 8, 16, 19}: the largest that
+//     still gives ~4 workgroups per CU over the launch, then a per-row merge;
+//     where 16 gives more than one residency round (4 workgroups per CU,
+//     kTargetBlocks) and 19 gives exactly one, MAXV = 19 (config 3: 8
+//     segments of 19 vectors per thread instead of 10 of 16, measured
+//     22.03 -> 21.45 us).
+static int plan_rows(int64_t rows, int64_t cols, int dt, bool few, Plan* p) {
   const int vec = dt == kF32 ? 4 : 8;
   const int64_t nv = (cols + 2 * (vec - 1)) / vec;  // covers any row misalignment
   static const int kOpts[3] = {16, 8, 4};
@@ -2007,10 +2016,12 @@ static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
   }
   for (int o = 0; o < 6; ++o) {  // whole-row parts, equal ones first
     const int np = 2 + o % 3;
-    if (o < 3 ? cols % np != 0 || rows * np > kPartsMaxBlocks
-              : rows * np < kUnevenMinBlocks || rows * np > kUnevenMaxBlocks)
-      continue;
     const int64_t nvh = (part_cols_of(cols, np, vec) + 2 * (vec - 1)) / vec;
+    if (o < 3 ? cols % np != 0 || rows * np > kPartsMaxBlocks
+              : rows * np < kUnevenMinBlocks || rows * np > kUnevenMaxBlocks ||
+                    nvh < (few ? kUnevenMinVecFew : dt == kBF16 ? kUnevenMinVecBf16 : 0) ||
+                    (few && (np == 4 || (dt == kBF16 && rows < kUnevenMinRowsFew))))
+      continue;
     if (nvh <= (int64_t)kNTS * 19) {
       p->nt = kNTS;
       p->maxv = nvh > (int64_t)kNTS * 16 ? 19 : 16;
@@ -2058,6 +2069,13 @@ static int plan_rows(int64_t rows, int64_t cols, int dt, Plan* p) {
 static size_t ws_bytes_for(int64_t rows, const Plan& p) {
   if (p.nseg <= 1) return 0;
   return (size_t)rows * p.nseg * kRun * sizeof(uint64_t);
+}
+
+// Workspace of the calls that read whole lists of 128 (sampler, shard candidates).
+static size_t list_ws_bytes(int64_t rows, int64_t cols, int dt) {
+  Plan p;
+  if (rows < 0 || cols <= 0 || (dt != kF32 && dt != kBF16) || plan_rows(rows, cols, dt, false, &p) != kOk) return 0;
+  return ws_bytes_for(rows, p);
 }
 
 template <int DT, int MAXV, int NT, bool SAMPLE>
@@ -2261,8 +2279,13 @@ size_t tallax_topk_workspace_size(int64_t rows, int64_t cols, int64_t k, int dty
   if (k < 1 || k > kMaxK || rows < 0 || cols <= 0) return 0;
   if (dtype == kI32) return topk_i32_ws(rows, cols);
   if (dtype != kF32 && dtype != kBF16) return 0;
-  if (plan_rows(rows, cols, dtype, &p) != kOk) return 0;
-  return ws_bytes_for(rows, p);
+  if (plan_rows(rows, cols, dtype, true, &p) != kOk) return 0;
+  const size_t few = ws_bytes_for(rows, p);
+  // k > 64 takes at most as many lists per row; the larger of both, so that a
+  // workspace for the largest k serves every smaller one
+  if (k <= kWave || plan_rows(rows, cols, dtype, false, &p) != kOk) return few;
+  const size_t all = ws_bytes_for(rows, p);
+  return all > few ? all : few;
 }
 
 int tallax_topk(const void* x, int dtype, int64_t rows, int64_t cols, int64_t k, void* out_vals,
@@ -2280,7 +2303,7 @@ int tallax_topk(const void* x, int dtype, int64_t rows, int64_t cols, int64_t k,
     return launch_topk_short(x, dtype, rows, cols, (int)k, ot, stream);
   }
   Plan p;
-  st = plan_rows(rows, cols, dtype, &p);
+  st = plan_rows(rows, cols, dtype, k <= kWave, &p);
   if (st) return st;
   const size_t need = ws_bytes_for(rows, p);
   if (workspace_bytes < need || (need && !workspace)) {
@@ -2317,7 +2340,7 @@ int tallax_topk_replace(const void* x, int dtype, int64_t rows, int64_t cols, in
     return launch_topk_short(x, dtype, rows, cols, (int)k, ot, stream);
   }
   Plan p;
-  st = plan_rows(rows, cols, dtype, &p);
+  st = plan_rows(rows, cols, dtype, k <= kWave, &p);
   if (st) return st;
   const size_t need = ws_bytes_for(rows, p);
   if (workspace_bytes < need || (need && !workspace)) {
@@ -2337,7 +2360,7 @@ int tallax_topk_replace(const void* x, int dtype, int64_t rows, int64_t cols, in
 }
 
 size_t tallax_sample_workspace_size(int64_t rows, int64_t vocab, int dtype) {
-  return tallax_topk_workspace_size(rows, vocab, kMaxK, dtype);
+  return list_ws_bytes(rows, vocab, dtype);
 }
 
 }  // extern "C"
@@ -2446,7 +2469,7 @@ static int fused_sample(const void* logits, int dtype, int64_t rows, int64_t voc
   if (!top_k || !top_p || !temperature || !rng_key || !out_tokens) { set_error("null pointer argument"); return kInvalidArgument; }
   if (rows == 0) return kOk;
   Plan p;
-  st = plan_rows(rows, vocab, dtype, &p);
+  st = plan_rows(rows, vocab, dtype, false, &p);
   if (st) return st;
   const size_t need = ws_bytes_for(rows, p);
   if (use_scratch) {
@@ -2482,7 +2505,7 @@ static int fused_sample(const void* logits, int dtype, int64_t rows, int64_t voc
 extern "C" {
 
 size_t tallax_shard_candidates_workspace_size(int64_t rows, int64_t cols, int dtype) {
-  return tallax_topk_workspace_size(rows, cols, kMaxK, dtype);
+  return list_ws_bytes(rows, cols, dtype);
 }
 
 int tallax_shard_candidates(const void* x, int dtype, int64_t rows, int64_t cols, int64_t col_offset,
@@ -2494,7 +2517,7 @@ int tallax_shard_candidates(const void* x, int dtype, int64_t rows, int64_t cols
   if (!candidates) { set_error("null pointer argument"); return kInvalidArgument; }
   if (rows == 0) return kOk;
   Plan p;
-  st = plan_rows(rows, cols, dtype, &p);
+  st = plan_rows(rows, cols, dtype, false, &p);
   if (st) return st;
   const size_t need = ws_bytes_for(rows, p);
   if (workspace_bytes < need || (need && !workspace)) {
@@ -2541,32 +2564,28 @@ int tallax_sample_from_candidates(const uint64_t* candidates, int64_t nlists, in
   return launch_status("tallax_sample_from_candidates");
 }
 
-int tallax_testing_select_plan(int64_t rows, int64_t cols, int dtype, int32_t* out) {
+int tallax_testing_select_route(int64_t rows, int64_t cols, int dtype, int few, int32_t* out) {
   if (!out || (dtype != kF32 && dtype != kBF16) || rows < 0 || cols <= 0) {
     set_error("bad arguments");
     return kInvalidArgument;
   }
   Plan p;
-  const int st = plan_rows(rows, cols, dtype, &p);
+  const int st = plan_rows(rows, cols, dtype, few != 0, &p);
   if (st) return st;
+  const int vec = dtype == kF32 ? 4 : 8;
   out[0] = p.nt;
   out[1] = p.maxv;
   out[2] = p.nseg;
   out[3] = (int32_t)p.vps;
+  out[4] = p.nt == kNTS && whole_row_edge(nullptr, cols, part_cols_of(cols, p.parts > 1 ? p.parts : 1, vec), 16 / vec);
   return kOk;
 }
 
-int tallax_testing_select_edge(int64_t rows, int64_t cols, int dtype, int32_t* out) {
-  if (!out || (dtype != kF32 && dtype != kBF16) || rows < 0 || cols <= 0) {
-    set_error("bad arguments");
-    return kInvalidArgument;
-  }
-  Plan p;
-  const int st = plan_rows(rows, cols, dtype, &p);
-  if (st) return st;
-  const int vec = dtype == kF32 ? 4 : 8;
-  out[0] = p.nt == kNTS && whole_row_edge(nullptr, cols, part_cols_of(cols, p.parts > 1 ? p.parts : 1, vec), 16 / vec);
-  return kOk;
+int tallax_testing_select_plan(int64_t rows, int64_t cols, int dtype, int32_t* out) {
+  int32_t r[5];
+  const int st = tallax_testing_select_route(rows, cols, dtype, 0, out ? r : nullptr);
+  if (st == kOk) memcpy(out, r, 4 * sizeof(int32_t));
+  return st;
 }
 
 int tallax_top_p_and_sample(const void* topk_logits, int dtype, const int32_t* topk_idx, int64_t rows,

@@ -157,3 +157,28 @@ def test_top_dynamic_k_path_hook_rejects_unknown_paths():
     st = _lib.LIB.tallax_testing_top_dynamic_k_path(1, 0, 8, 100, 1, 4, 8, 128, sched, 2, 0, 0, 0.0, 1, 1, 1, 1, 1,
                                                     1, 1 << 20, None, 7)
     assert st == _lib.INVALID_ARGUMENT and b"path" in _lib.LIB.tallax_last_error()
+
+
+def test_uneven_parts_route_without_gpu():
+    """Parts of rows that do not divide: both sides of each line, and a workspace
+    for the largest k that serves every smaller one."""
+    from tallax_amd import _lib
+    L, F, B = _lib.LIB, _lib.F32, _lib.BF16
+    # (rows, cols, dtype, k, sampler) -> parts, 0: segments
+    for rows, cols, dt, k, sample, parts in [
+            (63, 77827, F, 64, False, 0), (64, 77827, F, 64, False, 2), (128, 77827, F, 64, False, 2),
+            (129, 77827, F, 64, False, 0), (42, 100003, F, 50, False, 0), (43, 100003, F, 50, False, 3),
+            (32, 200003, F, 64, False, 0), (32, 200003, F, 65, False, 4), (31, 200003, F, 128, False, 0),
+            (43, 77827, F, 128, False, 3), (63, 200003, B, 64, False, 0), (64, 200003, B, 64, False, 2),
+            (43, 200003, B, 65, False, 3), (32, 200003, B, 128, True, 4), (32, 155653, B, 128, True, 0),
+            (43, 155653, B, 128, True, 3), (64, 155653, B, 128, True, 2)]:
+        p = _lib.select_plan(rows, cols, dt, k=k, sample=sample)
+        assert (p["segments"] if p["threads"] == 1024 else 0) == parts, (rows, cols, dt, k, p)
+    for rows in (32, 43, 64, 100):
+        for cols, dt in [(77827, F), (200003, F), (200003, B), (311299, B)]:
+            sizes = [L.tallax_topk_workspace_size(rows, cols, k, dt) for k in (1, 64, 65, 128)]
+            assert sizes == sorted(sizes) and sizes[0] > 0
+            for k in (50, 128):
+                assert sizes[-1] >= 1024 * rows * _lib.select_plan(rows, cols, dt, k=k, sample=False)["segments"]
+            assert L.tallax_sample_workspace_size(rows, cols, dt) == \
+                1024 * rows * _lib.select_plan(rows, cols, dt)["segments"]
