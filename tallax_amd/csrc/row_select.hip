@@ -1047,7 +1047,7 @@ void seg_select_kernel(SelArgs a) {
 
   // Filter pass; exact tie selection when a region overflows.  Control flow
   // is block-uniform.
-  int fill_from = kRun;  // candidates of a segment that has fewer than k
+  int fill_from = kRun;  // candidates of a segment that has fewer than k, and other elements
   {
     int wcnt = 0;
     rounds(wcnt);
@@ -1060,7 +1060,7 @@ void seg_select_kernel(SelArgs a) {
       int n = 0;
 #pragma unroll
       for (int q = 0; q < NW; ++q) n += sh.wc[q];
-      if (n < k) fill_from = n;
+      if (n < k && n < live_hi - live_lo) fill_from = n;  // (the list past n is zero)
     }
     if (overflow) {
       // its block sums order the reads of sh.wc above before the write below
