@@ -1,5 +1,5 @@
-// Exact top-k (k <= 128) of short rows (at most 2048 elements; 8192 for k <= 32
-// and many rows) for gfx950.
+// Exact top-k (k <= 128) of short rows (at most 2048 elements; with many rows
+// 8192 for k <= 16 and 4096 for k <= 32) for gfx950.
 //
 // A 1024-thread select workgroup per row (row_select.hip) spends its fixed
 // latency on a few hundred elements ([65536, 128] f32, k = 8: 1444 us), so short
@@ -29,7 +29,10 @@ constexpr int kLanesMaxK = 32;
 // networks: its fixed part grows with k (about 3, 4.5 and 7 us for lists of 8,
 // 16 and 32), its cost per row is the lowest, so the line lies where the rows
 // outweigh it (f32, others -> lanes, us).  k <= 8: [16, 256] 5.2 -> 3.4,
-// [256, 2048] 6.8 -> 6.3, [1024, 4096] 24.6 -> 10.6, but [256, 4096] 7.1 -> 9.6.
+// [256, 2048] 6.8 -> 6.3, [1024, 4096] 24.6 -> 10.6, but [256, 4096] 7.1 -> 9.6;
+// rows the one-wave networks of 64 and 128 slots take: [1, 64] 2.3 -> 3.4,
+// [2000, 64] 3.1 -> 3.6, [3000, 64] 3.5 -> 3.6, [6000, 64] 4.3 -> 3.7, [1, 128]
+// 3.0 -> 3.4, [512, 128] 3.6 -> 3.5, [2000, 128] 4.2 -> 3.7.
 // k <= 16: [512, 128] 3.7 -> 5.4, [65536, 128] 43 -> 18, [16, 256] 5.3 -> 4.1,
 // [256, 2048] 6.7 -> 7.1, [300, 2000] 11.6 -> 7.7.  k <= 32: [512, 128] 3.6 ->
 // 8.2, [65536, 128] 42 -> 26, [512, 2048] 12.2 -> 11.5, [1000, 2048] 22 -> 13,
@@ -38,7 +41,11 @@ constexpr int kLanesMaxK = 32;
 static bool topk_lanes_route(int64_t rows, int64_t cols, int k) {
   if (k > kLanesMaxK || cols > kLanesMaxCols) return false;
   if (cols <= 32) return true;
-  if (k <= 8) return cols <= 2048 || rows >= 1024;
+  if (k <= 8) {
+    if (cols <= 64) return rows >= 3072;
+    if (cols <= 128) return rows >= 512;
+    return cols <= 2048 || rows >= 1024;
+  }
   if (k <= 16) {
     if (cols <= 128) return rows * cols >= (int64_t)1 << 19;
     return cols <= 1024 || (cols <= 2048 ? rows > 256 : rows >= 1024);

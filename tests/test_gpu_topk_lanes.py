@@ -18,6 +18,7 @@ CASES = [
     (9, 256, 16), (8192, 256, 17), (5, 512, 8), (5, 513, 9), (4096, 512, 32), (3, 1024, 8), (3, 1025, 8),
     (2048, 1024, 32), (256, 2048, 16), (257, 2048, 16), (1024, 2048, 32), (1, 2047, 1), (1024, 2049, 8),
     (1023, 2049, 8), (1024, 4096, 32), (1025, 4097, 17), (1024, 8192, 8), (1024, 8191, 16), (1024, 8193, 8),
+    (3072, 64, 8), (3071, 64, 8), (3072, 33, 1), (3071, 33, 1), (512, 65, 8), (511, 65, 8), (512, 128, 8), (511, 128, 1),
 ]
 
 
