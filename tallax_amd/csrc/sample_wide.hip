@@ -97,7 +97,6 @@ struct SwArgs {
   const void* x;
   int64_t rows, cols;
   int k;         // candidates per row (K)
-  int vec;       // rows start 16-byte aligned: 8-element vector loads
   const int32_t* top_k;
   const float* top_p;
   const float* temperature;
@@ -110,57 +109,56 @@ struct SwArgs {
   float* out_vals;         // [rows, K] candidate values (f32), or null
 };
 
+// A row as whole aligned 16-byte vectors: slot i of `base` is column i - mis.
+// Every vector that is read holds a column of the row.
 template <int DT>
-__device__ __forceinline__ uint32_t sw_key_at(const char* rowp, int64_t i) {
-  if constexpr (DT == kBF16) return select_key(((uint32_t)((const uint16_t*)rowp)[i]) << 16);
-  else return select_key(((const uint32_t*)rowp)[i]);
-}
+struct SwRow {
+  const uint4* base;
+  int mis;
+  int64_t cols;
+};
 
-// Select keys of columns base .. base+7; returns the mask of those inside the row.
+// Select keys of slots s .. s + 7 (s a multiple of 8); returns the mask of those
+// inside the row.  (Element loads of rows that are not whole aligned vectors:
+// log-probabilities f32 [200, 50257], K = 256, 74 us with the read before them;
+// in whole vectors 49.)
 template <int DT>
-__device__ __forceinline__ uint32_t sw_load8(const char* rowp, int64_t cols, int64_t base, bool vec,
-                                             uint32_t (&k)[8]) {
-  if (vec && base + 8 <= cols) {
-    if constexpr (DT == kBF16) {
-      const uint4 w = *(const uint4*)(rowp + base * 2);
-      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+__device__ __forceinline__ uint32_t sw_load8(const SwRow<DT>& r, int64_t s, uint32_t (&k)[8]) {
+  const int64_t end = r.cols + r.mis;  // slots of the row: mis .. end - 1
+  uint32_t ws[8];
+  if constexpr (DT == kBF16) {
+    const uint4 w = s < end ? r.base[s / 8] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t d[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        k[2 * q] = select_key(ws[q] << 16);
-        k[2 * q + 1] = select_key(ws[q] & 0xFFFF0000u);
-      }
-    } else {
-      const uint4 w0 = *(const uint4*)(rowp + base * 4);
-      const uint4 w1 = *(const uint4*)(rowp + base * 4 + 16);
-      const uint32_t ws[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-      for (int q = 0; q < 8; ++q) k[q] = select_key(ws[q]);
+    for (int q = 0; q < 4; ++q) {
+      ws[2 * q] = d[q] << 16;
+      ws[2 * q + 1] = d[q] & 0xFFFF0000u;
     }
-    return 0xFFu;
+  } else {
+    const uint4 w0 = s < end ? r.base[s / 4] : make_uint4(0u, 0u, 0u, 0u);
+    const uint4 w1 = s + 4 < end ? r.base[s / 4 + 1] : make_uint4(0u, 0u, 0u, 0u);
+    ws[0] = w0.x; ws[1] = w0.y; ws[2] = w0.z; ws[3] = w0.w;
+    ws[4] = w1.x; ws[5] = w1.y; ws[6] = w1.z; ws[7] = w1.w;
   }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) k[q] = select_key(ws[q]);
+  if (s >= r.mis && s + 8 <= end) return 0xFFu;
   uint32_t m = 0;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int64_t i = base + q;
-    k[q] = 0u;
-    if (i < cols) {
-      k[q] = sw_key_at<DT>(rowp, i);
-      m |= 1u << q;
-    }
-  }
+  for (int q = 0; q < 8; ++q) m |= (s + q >= r.mis && s + q < end ? 1u : 0u) << q;
   return m;
 }
 
 // hist[(key >> dsh) & dmask] += 1 over the row's elements whose key >> fsh
 // equals fval (every element when !filt).
 template <int DT>
-__device__ __forceinline__ void sw_hist(const char* rowp, int64_t cols, bool vec, int nchunks, bool filt,
-                                        int fsh, uint32_t fval, int dsh, uint32_t dmask, int* hist) {
+__device__ __forceinline__ void sw_hist(const SwRow<DT>& row, int nchunks, bool filt, int fsh, uint32_t fval, int dsh,
+                                        uint32_t dmask, int* hist) {
 #pragma unroll 2
   for (int j = 0; j < nchunks; ++j) {
     const int64_t base = ((int64_t)j * kSwNT + threadIdx.x) * 8;
     uint32_t k[8];
-    const uint32_t m = sw_load8<DT>(rowp, cols, base, vec, k);
+    const uint32_t m = sw_load8<DT>(row, base, k);
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       if (((m >> q) & 1u) && (!filt || (k[q] >> fsh) == fval)) atomicAdd(&hist[(k[q] >> dsh) & dmask], 1);
@@ -188,7 +186,7 @@ __device__ __forceinline__ void sw_cross(const int* hist, int need, int* red, in
 // EDGE: rows that do not start 16-byte aligned or do not fill their last vector.
 // The register path reads them as whole aligned vectors too; the slots of the
 // first and last one outside the row become all-ones ([37, 47070] f32,
-// K = 512, on the element loads of the radix select before: 57 -> 22 us,
+// K = 512, on the radix select with element loads before: 57 -> 22 us,
 // [18, 110978] bf16 K = 1024 71 -> 24).
 template <int DT, bool EDGE>
 __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
@@ -222,18 +220,18 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
     row_temp = a.temperature[row];
   }
   const char* rowp = (const char*)a.x + (size_t)(row * a.cols) * ES;
-  const bool vec = a.vec != 0;
-  const int nchunks = (int)((a.cols + kSwChunk - 1) / kSwChunk);
 
   // --- register path: one read, the elements >= L -----------------------------
   constexpr int VEC = DT == kBF16 ? 8 : 4;
   constexpr int32_t kPosInf = DT == kBF16 ? 0x7F80 : 0x7F800000;  // +inf bits in the signed view
   const RowVec<ES> rv(rowp);
   const int mis = EDGE ? rv.mis : 0;  // slots of the first vector before the row
+  const SwRow<DT> rr = {rv.base, mis, a.cols};
+  const int nchunks = (int)((a.cols + mis + kSwChunk - 1) / kSwChunk);
   const int64_t nvec = (a.cols + mis + VEC - 1) / VEC;
   bool fast = nvec <= (int64_t)kSwNT * kSwV;  // block-uniform
   if (fast) {
-    const uint4* vb = EDGE ? rv.base : (const uint4*)rowp;
+    const uint4* vb = rv.base;
     uint4 raw[kSwV];
 #pragma unroll
     for (int j = 0; j < kSwV; ++j) {
@@ -250,6 +248,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
         asm volatile("" : "+v"(hj), "+v"(tj), "+v"(lo), "+v"(hi));
 #pragma unroll
         for (int j = 0; j < kSwV; ++j) {
+          if (!__ballot(hj == j || tj == j)) continue;  // wave-uniform: the masks are for two vectors of the row
           uint32_t d[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
           const int l0 = hj == j ? lo : 0, h0 = tj == j ? hi : VEC;
 #pragma unroll
@@ -483,7 +482,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
     const int dsh = ps == 0 ? 21 : ps == 1 ? 10 : 0;
     for (int i = t; i < kSwBins; i += kSwNT) s_hist[i] = 0;
     __syncthreads();
-    sw_hist<DT>(rowp, a.cols, vec, nchunks, ps > 0, dsh + bits, prefix, dsh, (1u << bits) - 1u, s_hist);
+    sw_hist<DT>(rr, nchunks, ps > 0, dsh + bits, prefix, dsh, (1u << bits) - 1u, s_hist);
     __syncthreads();
     sw_cross(s_hist, need, s_red, s_res);
     const int bin = s_res[0], above = s_res[1], cnt = s_res[2];
@@ -508,7 +507,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
   for (int j = 0; j < (fast ? 0 : nchunks); ++j) {
     const int64_t base = ((int64_t)j * kSwNT + t) * 8;
     uint32_t k[8];
-    const uint32_t m = sw_load8<DT>(rowp, a.cols, base, vec, k);
+    const uint32_t m = sw_load8<DT>(rr, base, k);
     uint32_t take = 0u, eq = 0u;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -533,7 +532,7 @@ __global__ __launch_bounds__(kSwNT) void sample_wide_kernel(SwArgs a) {
       const int q = __builtin_ctz(take);
       take &= take - 1u;
       const int pos = atomicAdd(&s_cnt, 1);
-      if (pos < kSwList) s_list[pos] = make_comp(k[q], (uint32_t)(base + q));
+      if (pos < kSwList) s_list[pos] = make_comp(k[q], (uint32_t)(base + q - mis));
     }
   }
   __syncthreads();
@@ -705,7 +704,7 @@ int tallax_sample_wide(const void* logits, int dtype, int64_t rows, int64_t voca
   SwArgs a = {};
   a.x = logits; a.rows = rows; a.cols = vocab; a.k = (int)max_k;
   const int es = dtype == kBF16 ? 2 : 4;
-  a.vec = ((uintptr_t)logits % 16 == 0) && ((vocab * es) % 16 == 0);
+  const bool whole = (uintptr_t)logits % 16 == 0 && (vocab * es) % 16 == 0;  // every row is whole aligned vectors
   a.top_k = top_k; a.top_p = top_p; a.temperature = temperature; a.rng_key = rng_key;
   a.dim0_offset = dim0_offset;
   const float rf = (float)replace_val;
@@ -713,10 +712,10 @@ int tallax_sample_wide(const void* logits, int dtype, int64_t rows, int64_t voca
   a.replace_in_dtype = dtype == kBF16 ? round_to_bf16(rf) : rf;
   a.out_tokens = out_tokens; a.out_idx = out_idx; a.out_vals = out_vals;
   if (dtype == kF32)
-    a.vec ? sample_wide_kernel<kF32, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
+    whole ? sample_wide_kernel<kF32, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
           : sample_wide_kernel<kF32, true><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
   else
-    a.vec ? sample_wide_kernel<kBF16, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
+    whole ? sample_wide_kernel<kBF16, false><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a)
           : sample_wide_kernel<kBF16, true><<<dim3((unsigned)rows), dim3(kSwNT), 0, stream>>>(a);
   return launch_status("tallax_sample_wide");
 }

@@ -36,3 +36,27 @@ def test_wide_edges_tokens(gpu):
     got = sampling.sample(key, to_dev(x, "bf16", gpu), meta, max_k=1024)
     want = O.sample((5, 6), host_values(x, "bf16"), topk, topp, temp, dtype="bf16", max_k=1024)
     assert np.array_equal(got.cpu().numpy(), want)
+
+
+# rows that end in the radix select, read as whole aligned vectors: row lengths
+# about a workgroup step of 8192 slots, ties at both edges of the row, the row
+# before and after full of larger values
+@pytest.mark.parametrize("cols,dtype", [(1031, "bf16"), (8185, "bf16"), (8191, "bf16"), (16386, "bf16"),
+                                        (200003, "bf16"), (1025, "f32"), (8190, "f32"), (8195, "f32"), (16387, "f32"),
+                                        (100001, "f32")])
+@pytest.mark.parametrize("k,kind", [(1024, "negative"), (512, "edges"), (700, "const"), (300, "masked5"),
+                                    (1000, "nan_heavy")])
+def test_wide_edges_radix(gpu, cols, dtype, k, kind):
+    from tallax_amd import sampling
+    print(f"wide edges radix cols={cols} {dtype} k={k} {kind}", flush=True)
+    if kind == "edges":   # more than 2048 ties, the first and last columns among them
+        x = -np.abs(np.random.default_rng(cols).standard_normal((9, cols))).astype(np.float32) - 1
+        x[:, :min(cols, 1500)] = -0.5
+        x[:, -min(cols, 1500):] = -0.5
+    else:
+        x = _make(9, cols, kind, seed=cols + k)
+    x[::2] += 100.0       # every second row lies above its neighbours
+    vals, idx = sampling.wide_top_k(to_dev(x, dtype, gpu), k)
+    wv, wi = O.top_k(host_values(x, dtype), k, dtype)
+    assert np.array_equal(idx.cpu().numpy(), wi)
+    assert np.array_equal(bits(vals.cpu().numpy()), bits(wv))
