@@ -364,8 +364,9 @@ __global__ __launch_bounds__(kMergeNT) void merge_runs_kernel(SortArgs a, const 
 // Multiway merge by splitters (rows of 3 to kBucketMaxRuns chunks): one pass
 // instead of ceil(log2 chunks) pairwise merge passes.
 //   * bucket_split_kernel, one workgroup per row: every G-th record of every
-//     sorted run is a sample (record (a + 1) G - 1 of a run); the samples (at most 4096) are sorted by a block bitonic
-//     network, and every m-th one of them in that order is a splitter s_k.
+//     sorted run is a sample (record (a + 1) G - 1 of a run); the samples (at
+//     most 4096) are sorted by a block bitonic network, and every m-th one of
+//     them in that order is a splitter s_k.
 //     For every splitter and run, the run's first position p_kj with a record
 //     >= s_k: the run's samples below s_k, c, put it in [c G, (c + 1) G), so a
 //     binary search of G records finds it.  Bucket k holds the records in
@@ -374,20 +375,22 @@ __global__ __launch_bounds__(kMergeNT) void merge_runs_kernel(SortArgs a, const 
 //     bucket never exceeds (m + runs) G records: m is chosen so that this is
 //     the bucket kernel's capacity.  The table holds every p_kj and each
 //     bucket's first output rank, sum_j p_kj.
-//     G is 64 where the samples fit: the finer they are, the fuller the buckets
-//     (79 % of the capacity at 13 runs against 58 % with G = 256).  Few rows take
-//     smaller buckets, so that they fill the chip.
+//     G is 64 where the samples fit: the finer they are, the more runs a bucket
+//     of 4096 records takes (m = 64 - runs samples: at 25 runs 39, buckets 61 %
+//     full on average; with 13 whole chunks and buckets of 8192, G = 64 fills 79 %
+//     and G = 256 58 %).  Few rows take smaller buckets, so that they fill the chip.
 //   * bucket_sort_kernel, one workgroup per (row, bucket): the bucket's part of
 //     every run, in tie order, sorted in LDS; the outputs (permutation, keys,
 //     gathered second key) are written from the bucket's first output rank.
 // Traffic: the chunk pass (4 bytes in, 8 out per element), then 8 in and the
 // outputs out: 28 bytes per element with keys and indices out, against 76 for
 // four pairwise merge passes at [1024, 201088].  There the three kernels take
-// 1000 + 272 + 1197 us: chunks bound by LDS (bank conflicts of the scattered
+// 990 + 271 + 1138 us: chunks bound by LDS (bank conflicts of the scattered
 // records), buckets by the latency of their loads and LDS steps.
 // ---------------------------------------------------------------------------
 constexpr int kBucketStride = 256;       // G: records between samples ...
 constexpr int kBucketStrideFine = 64;    // ... of rows of at most kSplitSamples * 64 elements
+constexpr int64_t kHalfChunkCols = 229376;  // longest rows sorted in half chunks
 constexpr int kBucketMaxRuns = 56;       // (m >= 8) + runs <= 64: buckets of at most 64 G = 16384 records
 constexpr int kSplitNT = 1024;
 constexpr int kSplitSamples = 4096;      // >= kBucketMaxRuns * kWideChunk / kBucketStride
@@ -499,14 +502,17 @@ __device__ __forceinline__ uint32_t bin_scale(uint32_t range) {
 // in its bin, a scan the bins' starts, and after one move through LDS a
 // record's rank is its bin's start + the smaller records of its bin.  That is
 // one pass and five barriers, against three to four radix passes of five
-// ([1024, 201088] f32, buckets of 8192: 1792 -> 1210 us; of 4096, four
-// workgroups to a CU: 994).
-// bf16 keys, key ranges of few values and bunched keys pile up in the bins and
-// take the stable radix sort on the key.
+// ([1024, 201088] f32 in whole chunks, buckets of 8192: 1792 -> 1210 us; of 4096,
+// four workgroups to a CU: 994; in half chunks 1185, without
+// spilled registers, which one order of slots throughout removed, 1138).  bf16 keys, key
+// ranges of few values and bunched keys pile up in the bins and take the stable
+// radix sort on the key; the records are held in its slot order from the start.
+// f32 rows of few values pay the counting pass for nothing: whole sort [64, 50257]
+// of ten values 147 us without bins and in whole chunks, 168 now ([64, 201088]
+// 360 / 302), of bf16 values held in f32 122 / 136 (327 / 290).
 template <int NT, int E, int DT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(E <= 16 ? 4 : 2, 8)))
-void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
-                                                                const int32_t* table) {
+void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs, const int32_t* table) {
   constexpr int NW = NT / kWave;
   constexpr int BINS = bucket_bins(NT, E);  // 0: the radix sort only
   constexpr int CAP = E * NT;
@@ -545,7 +551,8 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
   const int n = s_off[R];  // at most CAP (the split's bound)
   if (n > CAP) return;     // never taken; keeps a broken table from writing past the LDS buffer
   const int64_t o0 = tp[(bp.K + 1) * R + k];
-  uint32_t kmin = ~0u, kmax = 0u;
+  // a thread's slots, as the radix sort numbers them: ascending
+  auto slot_of = [&](int r) -> int { return w * (E * kWave) + r * kWave + l; };
   uint64_t v[E];
   {
     // a row's records span less than 2^32 bytes: 32-bit offsets from its start
@@ -553,116 +560,127 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
     int i = 0;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const int L = r * NT + t;
+      const int L = slot_of(r);
       v[r] = ~0ull;
       if (L < n) {
-        while (s_off[i + 1] <= L) ++i;  // a thread's slots ascend
+        while (s_off[i + 1] <= L) ++i;
         v[r] = *(const uint64_t*)(rr + (s_src[i] + (uint32_t)L) * 8u);
       }
     }
+  }
+  bool spread = false;  // block-uniform: the bins order the bucket
+  uint32_t kmin = ~0u, scale = 0u;
+  auto bin_of = [&](uint64_t x) -> uint32_t { return __umulhi((uint32_t)(x >> 32) - kmin, scale); };
+  const uint16_t* start = (const uint16_t*)bins;
+  if constexpr (DT != kBF16 && BINS > 0) {
+    uint32_t kmax = 0u;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      if (r * NT + t < n) {
+      if (slot_of(r) < n) {
         const uint32_t key = (uint32_t)(v[r] >> 32);
         kmin = key < kmin ? key : kmin;
         kmax = key > kmax ? key : kmax;
       }
     }
-  }
-  kmin = wave_min_u32(kmin);
-  kmax = wave_max_u32(kmax);
-  if (l == 0) {
-    red[0][w] = kmin;
-    red[1][w] = kmax;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    kmin = red[0][i] < kmin ? red[0][i] : kmin;
-    kmax = red[1][i] > kmax ? red[1][i] : kmax;
-  }
-  kmin = __builtin_amdgcn_readfirstlane(kmin);
-  kmax = __builtin_amdgcn_readfirstlane(kmax);
-  const uint32_t scale = bin_scale<BINS>(kmax - kmin);
-  auto bin_of = [&](uint64_t x) -> uint32_t { return __umulhi((uint32_t)(x >> 32) - kmin, scale); };
-  uint32_t bin_most = ~0u;
-  uint32_t pb[E];  // place in the bin << 16 | bin
-  if constexpr (DT != kBF16 && BINS > 0) {
-  if (kmax - kmin >= (uint32_t)n / 4u) {  // block-uniform
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-      pb[r] = 0u;
-      if (r * NT + t < n) {
-        const uint32_t b = bin_of(v[r]), sh = (b & 1u) * 16u;
-        pb[r] = ((atomicAdd(&bins[b >> 1], 1u << sh) >> sh) << 16) | b;
-      }
-    }
-    __syncthreads();
-    constexpr int PW = BINS / 2 / NT;  // words per thread
-    uint32_t cw[PW], most = 0u;
-    int sum = 0;
-#pragma unroll
-    for (int q = 0; q < PW; ++q) {
-      cw[q] = bins[t * PW + q];
-      const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
-      sum += (int)(lo + hi);
-      most = max(most, max(lo, hi));
-    }
-    int tot;
-    const int pre = wave_exscan_i32(sum, tot);
-    most = wave_max_u32(most);
+    kmin = wave_min_u32(kmin);
+    kmax = wave_max_u32(kmax);
     if (l == 0) {
-      wsum[w] = (uint32_t)tot;
-      red[0][w] = most;
+      red[0][w] = kmin;
+      red[1][w] = kmax;
     }
     __syncthreads();
-    uint32_t run = (uint32_t)pre;
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
-      run += i < w ? wsum[i] : 0u;
-      most = max(most, red[0][i]);
+      kmin = red[0][i] < kmin ? red[0][i] : kmin;
+      kmax = red[1][i] > kmax ? red[1][i] : kmax;
     }
+    kmin = __builtin_amdgcn_readfirstlane(kmin);
+    kmax = __builtin_amdgcn_readfirstlane(kmax);
+    scale = bin_scale<BINS>(kmax - kmin);
+    if (kmax - kmin >= (uint32_t)n / 4u) {  // block-uniform: else few values
+      uint32_t pb[E];  // place in the bin << 16 | bin
 #pragma unroll
-    for (int q = 0; q < PW; ++q) {
-      const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
-      bins[t * PW + q] = run | ((run + lo) << 16);  // the bins' starts, below 2^16
-      run += lo + hi;
+      for (int r = 0; r < E; ++r) {
+        pb[r] = 0u;
+        if (slot_of(r) < n) {
+          const uint32_t b = bin_of(v[r]), sh = (b & 1u) * 16u;
+          pb[r] = ((atomicAdd(&bins[b >> 1], 1u << sh) >> sh) << 16) | b;
+        }
+      }
+      __syncthreads();
+      constexpr int PW = BINS / 2 / NT;  // words per thread
+      uint32_t cw[PW], most = 0u;
+      int sum = 0;
+#pragma unroll
+      for (int q = 0; q < PW; ++q) {
+        cw[q] = bins[t * PW + q];
+        const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
+        sum += (int)(lo + hi);
+        most = max(most, max(lo, hi));
+      }
+      int tot;
+      const int pre = wave_exscan_i32(sum, tot);
+      most = wave_max_u32(most);
+      if (l == 0) {
+        wsum[w] = (uint32_t)tot;
+        red[0][w] = most;
+      }
+      __syncthreads();
+      uint32_t run = (uint32_t)pre;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        run += i < w ? wsum[i] : 0u;
+        most = max(most, red[0][i]);
+      }
+      spread = __builtin_amdgcn_readfirstlane(most) <= kBinMost;
+      if (spread) {
+#pragma unroll
+        for (int q = 0; q < PW; ++q) {
+          const uint32_t lo = cw[q] & 0xFFFFu, hi = cw[q] >> 16;
+          bins[t * PW + q] = run | ((run + lo) << 16);  // the bins' starts, below 2^16
+          run += lo + hi;
+        }
+        if (t == 0) bins[BINS / 2] = (uint32_t)n;  // the end of the last bin
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < E; ++r)
+          if (slot_of(r) < n) buf[start[pb[r] & 0xFFFFu] + (pb[r] >> 16)] = v[r];
+        if (t < kBucketPad) buf[n + t] = ~0ull;  // read past the last bin: larger than any record
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = slot_of(r) < n ? buf[slot_of(r)] : ~0ull;
+      }
     }
-    if (t == 0) bins[BINS / 2] = (uint32_t)n;  // the end of the last bin
-    bin_most = __builtin_amdgcn_readfirstlane(most);
+    __syncthreads();  // red is read, and the radix sort clears its counters over the bins
   }
-  }
-  const bool spread = bin_most <= kBinMost;  // block-uniform
-  const uint16_t* start = (const uint16_t*)bins;
-  __syncthreads();
-  if (spread) {
-#pragma unroll
-    for (int r = 0; r < E; ++r)
-      if (r * NT + t < n) buf[start[pb[r] & 0xFFFFu] + (pb[r] >> 16)] = v[r];
-    if (t < kBucketPad) buf[n + t] = ~0ull;  // read past the last bin: larger than any record
-  } else {
-    // the slots in the radix sort's order, then back
-#pragma unroll
-    for (int r = 0; r < E; ++r)
-      if (r * NT + t < n) buf[r * NT + t] = v[r];
-    __syncthreads();
+  if (!spread) {
+    // the digits in which no key varies are skipped: all but two or three of a
+    // tied bucket's, the low two of bf16 values held in f32.  (From the smallest
+    // and largest key alone, every digit below their first difference was
+    // sorted: [64, 201088] f32 holding bf16 values 328 -> 412 us.)
+    uint32_t kand = ~0u, kor = 0u;
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const int L = w * (E * kWave) + r * kWave + l;
-      v[r] = L < n ? buf[L] : ~0ull;
+      if (slot_of(r) < n) {
+        kand &= (uint32_t)(v[r] >> 32);
+        kor |= (uint32_t)(v[r] >> 32);
+      }
     }
-    __syncthreads();  // the radix sort clears its counters over the bins and moves over buf
-    uint32_t varying = kmin == kmax ? 0u : 0xFFFFFFFFu >> __clz((int)(kmin ^ kmax));
-    if (DT == kBF16) varying &= 0xFFFF0000u;  // the low order bits of a bf16 key follow from the high
-    radix_sort_slots<E, NT>(v, buf, hist, wsum, varying, n);
+    kand = wave_and_u32(kand);
+    kor = wave_or_u32(kor);
+    if (l == 0) {
+      red[0][w] = kand;
+      red[1][w] = kor;
+    }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-      const int L = w * (E * kWave) + r * kWave + l;
-      if (L < n) buf[L] = v[r];
+    for (int i = 0; i < NW; ++i) {
+      kand &= red[0][i];
+      kor |= red[1][i];
     }
+    // the low order bits of a bf16 key follow from the high
+    radix_sort_slots<E, NT>(v, buf, hist, wsum, (kand ^ kor) & (DT == kBF16 ? 0xFFFF0000u : ~0u), n);
   }
-  __syncthreads();
   // outputs at o0 + rank: the source column, the sorted key and the gathered
   // second key (32-bit offsets from the bucket's first output)
   const int64_t ob = base + o0;
@@ -687,9 +705,9 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
   if (!a.perm_in && !a.aux_out) {
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const int L = r * NT + t;
+      const int L = slot_of(r);
       if (L >= n) continue;
-      const uint64_t x = buf[L];
+      const uint64_t x = v[r];
       const uint32_t k0 = rank_of(x, L);
       po[k0] = (int32_t)((uint32_t)x ^ tmask);
       if (a.key_out) store_sorted(ko, a.key_out_dtype, DT, k0, (uint32_t)(x >> 32) ^ dmask);
@@ -701,11 +719,11 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
   uint32_t rank[E], col[E];
 #pragma unroll
   for (int r = 0; r < E; ++r) {
-    const int L = r * NT + t;
+    const int L = slot_of(r);
     rank[r] = 0u;
     col[r] = 0u;
     if (L >= n) continue;
-    const uint64_t x = buf[L];
+    const uint64_t x = v[r];
     rank[r] = rank_of(x, L);
     const uint32_t pos = (uint32_t)x ^ tmask;
     col[r] = a.perm_in ? (uint32_t)a.perm_in[base + pos] : pos;
@@ -713,21 +731,21 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs,
   }
 #pragma unroll
   for (int r = 0; r < E; ++r)
-    if (r * NT + t < n) po[rank[r]] = (int32_t)col[r];
+    if (slot_of(r) < n) po[rank[r]] = (int32_t)col[r];
   if (a.aux_out) {
     uint32_t u[E];
     if (a.aux_dtype == kBF16) {
 #pragma unroll
       for (int r = 0; r < E; ++r)
-        u[r] = r * NT + t < n ? key_bits_at<kBF16>(a.aux, base + col[r]) : 0u;
+        u[r] = slot_of(r) < n ? key_bits_at<kBF16>(a.aux, base + col[r]) : 0u;
     } else {
 #pragma unroll
       for (int r = 0; r < E; ++r)
-        u[r] = r * NT + t < n ? key_bits_at<kF32>(a.aux, base + col[r]) : 0u;
+        u[r] = slot_of(r) < n ? key_bits_at<kF32>(a.aux, base + col[r]) : 0u;
     }
 #pragma unroll
     for (int r = 0; r < E; ++r)
-      if (r * NT + t < n)
+      if (slot_of(r) < n)
         store_sorted(a.aux_out, a.aux_out_dtype, a.aux_dtype, ob + rank[r], order_from_bits(u[r], a.aux_dtype));
   }
 }
@@ -917,13 +935,16 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
     return kUnsupported;
   }
   // Rows whose samples fit at a stride of 64 take half chunks, two workgroups to a
-  // CU: one's LDS work covers the other's barriers (f32 [1024, 201088], chunks
-  // 1340 -> 1000 us; twice the runs cost the splitters 177 -> 272 and the buckets
-  // 994 -> 1197; in all 2510 -> 2405, [300, 50257] i32 282 -> 225, [14, 60833]
-  // 60 -> 55, bf16 [64, 131072] 140 -> 123).  Rows of two whole chunks stay on
-  // the merge pass: their workspace holds no splitter table.
-  const bool small = cols > 2 * kWideChunk && cols <= (int64_t)kSplitSamples * kBucketStrideFine;
-  const int chunk = small ? kWideChunk / 2 : kWideChunk;
+  // CU: one's LDS work covers the other's barriers (f32 [1024, 201088], whole / half
+  // chunks: 2510 / 2405 us, chunks 1340 / 1000, splitters 177 / 272, buckets
+  // 994 / 1197; [300, 50257] i32 282 / 225, [14, 60833] 60 / 55, bf16 [64, 131072]
+  // 140 / 123).  Past kHalfChunkCols twice the runs cost the splitters and the
+  // buckets more than the chunks gain (f32, [16, 229377] 98 / 109, [50, 262144]
+  // 228 / 245, [4, 262144] 89 / 96; [4, 201088] 83 / 73).  Rows of two whole chunks
+  // stay on the merge pass: their workspace holds no splitter table.
+  const bool fine = cols > 2 * kWideChunk && cols <= (int64_t)kSplitSamples * kBucketStrideFine;
+  const bool half = fine && cols <= kHalfChunkCols;
+  const int chunk = half ? kWideChunk / 2 : kWideChunk;
   const int64_t nchunks = (cols + chunk - 1) / chunk;
   const int64_t tiles = (cols + kMergeTile - 1) / kMergeTile;
   if (rows * tiles > 2147483647 || rows * nchunks > 2147483647) {
@@ -952,8 +973,8 @@ int launch_sort_wide(const SortArgs& a, int64_t rows, void* ws, size_t ws_bytes,
     BucketPlan bp;
     bp.runs = (int)nchunks;
     bp.chunk = chunk;
-    bp.G = small ? kBucketStrideFine : kBucketStride;
-    bp.cap = small ? 4096 : bp.runs <= 24 ? 8192 : 16384;
+    bp.G = fine ? kBucketStrideFine : kBucketStride;
+    bp.cap = fine ? 4096 : bp.runs <= 24 ? 8192 : 16384;
     bp.samples = 0;
     for (int j = 0; j < bp.runs; ++j) bp.samples += run_len(cols, bp.chunk, j) / bp.G;
     bp.m = bp.cap / bp.G - bp.runs;  // (m + runs) G = capacity

@@ -71,3 +71,46 @@ def test_bucket_sort_int_and_second_key(gpu, rows, descending):
     want, _ = O.sort([b], 1, return_argsort=True, descending=descending, dtypes=["i32"])
     for g, w in zip(got, want):
         assert np.array_equal(g.cpu().numpy(), w)
+
+
+# every instance of the bucket kernel (4096 records, 8192, 16384) and the first
+# row past the longest sorted in half chunks, with a second key and a permutation
+# to compose; keys that spread over the bins, keys that tie, and bf16 values held
+# in f32 (low digits that no key varies in)
+@pytest.mark.parametrize("cols", [50257, 229377, 262145, 393217])
+@pytest.mark.parametrize("first", ["i32", "ties", "bf16"])
+@pytest.mark.parametrize("second", ["f32", "bf16"])
+@pytest.mark.parametrize("descending", [False, True])
+def test_bucket_sort_two_keys(gpu, cols, first, second, descending):
+    from tallax_amd import tax
+    print(f"bucket sort two keys cols={cols} {first} {second} desc={descending}", flush=True)
+    rng = np.random.default_rng(cols)
+    rows = 3
+    b = np.round(rng.standard_normal((rows, cols)) * 64).astype(np.float32) / 8
+    db, bt = to_dev(b, second, gpu), O.round_to_dtype(b, second)
+    if first == "bf16":   # not a packed key: it comes back as float32
+        a = rng.standard_normal((rows, cols)).astype(np.float32)
+        da, a, dt = to_dev(a, "bf16", gpu), O.round_to_dtype(a, "bf16"), "bf16"
+    else:
+        lim = 4 if first == "ties" else 2**31 - 1
+        a = rng.integers(-lim, lim, (rows, cols), dtype=np.int64).astype(np.int32)
+        da, dt = torch.from_numpy(a).to(gpu), "i32"
+    got = tax.sort([da, db], num_keys=2, return_argsort=True, descending=descending)
+    want, _ = O.sort([a, bt], 2, return_argsort=True, descending=descending, dtypes=[dt, second])
+    for g, w in zip(got, want):
+        g = g.cpu().numpy() if g.dtype != torch.bfloat16 else g.float().cpu().numpy()
+        assert np.array_equal(g if g.dtype == np.int32 else bits(g), w if w.dtype == np.int32 else bits(w))
+
+
+@pytest.mark.parametrize("cols", [32769, 229376, 229377, 262144, 300001, 393217])
+@pytest.mark.parametrize("descending", [False, True])
+def test_bucket_sort_coarse_floats(gpu, cols, descending):
+    """bf16 values held in float32, of both signs: the low digits are all zeros or
+    all ones, and the radix sort skips what no key of a bucket varies in."""
+    from tallax_amd import tax
+    print(f"bucket sort coarse floats cols={cols} desc={descending}", flush=True)
+    x = O.round_to_dtype(np.random.default_rng(cols).standard_normal((3, cols)).astype(np.float32) * 3, "bf16")
+    got = tax.sort(torch.from_numpy(x).to(gpu), num_keys=1, is_stable=True, return_argsort=True, descending=descending)
+    want, _ = O.sort([x], 1, is_stable=True, return_argsort=True, descending=descending, dtypes=["f32"])
+    assert np.array_equal(got[1].cpu().numpy(), want[1])
+    assert np.array_equal(bits(got[0].cpu().numpy()), bits(want[0]))
