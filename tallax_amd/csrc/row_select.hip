@@ -942,7 +942,7 @@ void seg_select_kernel(SelArgs a) {
   // fewer than k of them (constrained decoding: -inf but a few) takes the rest
   // of its list by class (fill_ineligible) instead of collecting its -inf
   // elements, which overflowed every region into the tie selection (sampler
-  // [67, 151937] f32, three rows in four masked: 65.5 -> 25.5 us).
+  // [200, 100003] f32, three rows in four masked: 104 -> 32 us).
   const uint32_t thr = L > kFloor ? L : kFloor;
 
   // ---- flags: vectors whose maximum may reach thr ------------------------------

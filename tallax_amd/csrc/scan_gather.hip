@@ -325,8 +325,9 @@ __global__ __launch_bounds__(kScanNT) void cumsum_rows_kernel(const T* __restric
     run = run_sh;
 #pragma unroll
     for (int h = 0; h < 8; ++h) c[h] = nx[h];
-    // no third barrier: the next writes of tsum, carry and run_sh follow the
-    // next chunk's first barrier, which every wave reaches after its reads
+    // no third barrier: wave 0 reads tsum before this chunk's second barrier, and
+    // the next chunk writes it after that one; carry and run_sh are written after
+    // the next chunk's first barrier, which every wave reaches after its reads
   }
 }
 
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(kChainNT) void cumsum_chain_kernel(T* __restrict__ 
     }
     __syncthreads();
     const int ns = (nb + kChainRun - 1) / kChainRun;  // stretches of a line
-    if (ns == 1) {  // at most 32 tiles, the line's only block: the repeat below is the chain
+    if (ns == 1) {  // at most 32 tiles, the line's only or last block: the repeat below is the chain
       if (j0 < gl) start[j0] = acc;
     } else if (j0 < gl) {
       // the running total before each stretch: one dependent add per tile, the

@@ -167,9 +167,9 @@ __device__ __attribute__((noinline)) uint64_t pf_kth_comp(const uint4* base, int
 // other sorts.  SUMM: group summary and histogram threshold (rows of at most
 // kPfMaxGroups groups); otherwise per-thread top-4 and a full second read.
 // SHORT: rows whose groups are too few to bound the candidates (the launch's
-// rule); every such row takes pf_kth_comp.  The other instances keep the
-// bisection for rows of heavy ties: a call there costs the streaming loop
-// registers ([1024, 201088] 194 -> 202 us, 207 inlined).
+// rule); those whose candidates overflow the pool take pf_kth_comp.  The other
+// instances keep the bisection for rows of heavy ties: a call there costs the
+// streaming loop registers ([1024, 201088] 194 -> 202 us, 207 inlined).
 template <bool SUMM, bool SHORT>
 __global__ __launch_bounds__(kPfNT) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void softmax_topk_kernel(PfArgs a) {

@@ -14,9 +14,13 @@
 // unique, so any correct sort of them gives exactly that order, and two
 // sorted runs merge without a stability rule.
 //   1. sort_chunks_kernel: one 512-thread workgroup sorts each 16384- or
-//      8192-record chunk of a row in LDS (a stable LSD radix sort on the key, 8-bit
-//      digits) and writes the sorted run to the workspace.
-//   2. merge_runs_kernel, ceil(log2(chunks)) passes: runs of length L are
+//      8192-record chunk of a row in LDS (a stable LSD radix sort on the key,
+//      8-bit digits) and writes the sorted run to the workspace.
+//   2. Rows of 3 to kBucketMaxRuns chunks: bucket_split_kernel cuts the key
+//      range into buckets by samples of the runs, and bucket_sort_kernel orders
+//      each bucket in LDS and writes the outputs.  One pass over the records.
+//   3. Rows of two chunks, or more than that: merge_runs_kernel,
+//      ceil(log2(chunks)) passes.  Runs of length L are
 //      merged pairwise into runs of 2L, ping-ponging between two workspace
 //      buffers.  A workgroup produces 4096 consecutive outputs of one pair:
 //      two waves find the tile's start and end on the merge path with a
@@ -26,8 +30,8 @@
 //      and merges sequentially, and the tile leaves through LDS as coalesced
 //      stores.  The last pass writes the permutation, the decoded keys and
 //      the gathered second key instead of records.
-// Every pass reads and writes each record once (16 bytes per element per
-// pass); no kernel waits on another workgroup.
+// Every merge pass reads and writes each record once (16 bytes per element per
+// pass), the buckets read it once; no kernel waits on another workgroup.
 #include <stdint.h>
 
 #include "tallax_hip.h"
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(kChunkNT) void sort_chunks_kernel(SortArgs a, int n
   constexpr int CH = E * kChunkNT;                     // records of a chunk
   extern __shared__ __align__(16) unsigned char smem[];
   uint64_t* buf = (uint64_t*)smem;                     // CH records
-  uint32_t* hist = (uint32_t*)(buf + CH);      // 256 * HS counters
+  uint32_t* hist = (uint32_t*)(buf + CH);              // 256 * (NW + 1) counters
   __shared__ uint32_t wsum[NW];
   __shared__ uint32_t red[2][NW];
   const int t = threadIdx.x, l = lane_id(), w = t / kWave;
@@ -503,10 +507,10 @@ __device__ __forceinline__ uint32_t bin_scale(uint32_t range) {
 // record's rank is its bin's start + the smaller records of its bin.  That is
 // one pass and five barriers, against three to four radix passes of five
 // ([1024, 201088] f32 in whole chunks, buckets of 8192: 1792 -> 1210 us; of 4096,
-// four workgroups to a CU: 994; in half chunks 1185, without
-// spilled registers, which one order of slots throughout removed, 1138).  bf16 keys, key
-// ranges of few values and bunched keys pile up in the bins and take the stable
-// radix sort on the key; the records are held in its slot order from the start.
+// four workgroups to a CU: 994; in half chunks 1185, and 1138 with one order of
+// slots throughout, which left no register spilled).  bf16 keys, key ranges of
+// few values and bunched keys pile up in the bins and take the stable radix sort
+// on the key; the records are held in its slot order from the start.
 // f32 rows of few values pay the counting pass for nothing: whole sort [64, 50257]
 // of ten values 147 us without bins and in whole chunks, 168 now ([64, 201088]
 // 360 / 302), of bf16 values held in f32 122 / 136 (327 / 290).

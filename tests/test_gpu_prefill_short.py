@@ -20,8 +20,11 @@ def _rows(rng, cols):
     return x
 
 
-# groups of 16 elements below, at and above 1.25 k; k = cols; short odd rows
+# groups of 16 elements below, at and above 1.25 k (40941 columns: 2559 groups, the
+# last short row at k = 2048; 40942: 2560), rows whose ties overflow the candidate
+# pool on both sides; k = cols; short odd rows
 @pytest.mark.parametrize("cols,k", [(10926, 1616), (8193, 2048), (16384, 2048), (40959, 2048), (40961, 2048),
+                                    (40941, 2048), (40942, 2048), (20461, 1024), (20462, 1024),
                                     (2048, 2048), (517, 300), (1, 1), (33, 2), (5000, 256)])
 def test_short_rows(gpu, cols, k):
     from tallax_amd import prefill
