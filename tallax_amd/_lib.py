@@ -186,7 +186,8 @@ def select_plan(rows: int, cols: int, dtype: int, k: int = 128, sample: bool = T
     whole-row parts (1024 threads, `segments` = parts) or 256-thread segments.
     Rows of several segments or parts finish in seg_merge64_pair_kernel (two
     lists) or seg_merge64_kernel for top-k with k <= 64 (no sampler), else in
-    seg_merge_kernel."""
+    seg_merge_kernel.  "(parts)" stands for the whole-row kernel's instance for
+    parts (its last template argument, false where it is not given)."""
     out = (ctypes.c_int32 * 5)()
     few = not sample and k <= 64
     check(LIB.tallax_testing_select_route(rows, cols, dtype, int(few), out), "select_plan")
