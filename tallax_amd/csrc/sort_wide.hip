@@ -53,9 +53,9 @@ constexpr uint32_t kTieMask = 0x7FFFFFFFu;
 static_assert((2 * kWideChunk) % kMergeTile == 0, "a merge tile never straddles two pairs of runs");
 static_assert(kChunkE * kChunkNT == kWideChunk, "whole chunks per workgroup");
 
-// Stable LSD radix sort by the key (the records' high 32 bits) of the E x NT
-// records a workgroup holds in registers in slot order, slot
-// (E * 64) w + 64 r + l being record r of lane l of wave w; 8-bit digits, the
+// Stable LSD radix sort by the key (the records' high 32 bits) of the per x NT
+// records (per <= E) a workgroup holds in registers in slot order, slot
+// (per * 64) w + 64 r + l being record r of lane l of wave w; 8-bit digits, the
 // digits in which no key varies skipped.  Slots n and above hold all-ones
 // records, which stay last: waves wholly past n neither count nor move theirs.
 // buf holds E * NT records, hist 256 * (NT / 64 + 1) counters.  Every thread
@@ -71,12 +71,12 @@ static_assert(kChunkE * kChunkNT == kWideChunk, "whole chunks per workgroup");
 //     pass reads them back in slot order.
 template <int E, int NT>
 __device__ __forceinline__ void radix_sort_slots(uint64_t (&v)[E], uint64_t* buf, uint32_t* hist, uint32_t* wsum,
-                                                 uint32_t varying, int n) {
+                                                 uint32_t varying, int n, int per = E) {
   constexpr int NW = NT / kWave;
   constexpr int HS = NW + 1;  // counter stride per digit
   static_assert(256 * NW == 4 * NT, "four counters per thread in the scan");
   const int t = threadIdx.x, l = lane_id(), w = t / kWave;
-  const bool live = w * (E * kWave) < n;  // wave-uniform: the wave holds a slot below n
+  const bool live = w * (per * kWave) < n;  // wave-uniform: the wave holds a slot below n
 #pragma unroll 1
   for (int sh = 0; sh < 32; sh += 8) {
     if (((varying >> sh) & 0xFFu) == 0u) continue;  // every key has this digit: the pass is the identity
@@ -86,8 +86,10 @@ __device__ __forceinline__ void radix_sort_slots(uint64_t (&v)[E], uint64_t* buf
     if (live) {
 #pragma unroll
       for (int r = 0; r < E; ++r) {
-        const uint32_t d = (uint32_t)(v[r] >> (32 + sh)) & 0xFFu;
-        rk[r] = atomicAdd(&hist[d * HS + w], 1u);
+        if (r < per) {
+          const uint32_t d = (uint32_t)(v[r] >> (32 + sh)) & 0xFFu;
+          rk[r] = atomicAdd(&hist[d * HS + w], 1u);
+        }
       }
     }
     __syncthreads();  // every count is in
@@ -112,15 +114,17 @@ __device__ __forceinline__ void radix_sort_slots(uint64_t (&v)[E], uint64_t* buf
     if (live) {
 #pragma unroll
       for (int r = 0; r < E; ++r) {
-        const uint32_t d = (uint32_t)(v[r] >> (32 + sh)) & 0xFFu;
-        buf[hist[d * HS + w] + rk[r]] = v[r];
+        if (r < per) {
+          const uint32_t d = (uint32_t)(v[r] >> (32 + sh)) & 0xFFu;
+          buf[hist[d * HS + w] + rk[r]] = v[r];
+        }
       }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < E; ++r) {
-      const int L = w * (E * kWave) + r * kWave + l;
-      v[r] = L < n ? buf[L] : ~0ull;
+      const int L = w * (per * kWave) + r * kWave + l;
+      v[r] = r < per && L < n ? buf[L] : ~0ull;
     }
   }
 }
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(kMergeNT) void merge_runs_kernel(SortArgs a, const 
 // Traffic: the chunk pass (4 bytes in, 8 out per element), then 8 in and the
 // outputs out: 28 bytes per element with keys and indices out, against 76 for
 // four pairwise merge passes at [1024, 201088].  There the three kernels take
-// 990 + 271 + 1138 us: chunks bound by LDS (bank conflicts of the scattered
+// 991 + 271 + 983 us: chunks bound by LDS (bank conflicts of the scattered
 // records), buckets by the latency of their loads and LDS steps.
 // ---------------------------------------------------------------------------
 constexpr int kBucketStride = 256;       // G: records between samples ...
@@ -507,13 +511,14 @@ __device__ __forceinline__ uint32_t bin_scale(uint32_t range) {
 // record's rank is its bin's start + the smaller records of its bin.  That is
 // one pass and five barriers, against three to four radix passes of five
 // ([1024, 201088] f32 in whole chunks, buckets of 8192: 1792 -> 1210 us; of 4096,
-// four workgroups to a CU: 994; in half chunks 1185, and 1138 with one order of
-// slots throughout, which left no register spilled).  bf16 keys, key ranges of
-// few values and bunched keys pile up in the bins and take the stable radix sort
-// on the key; the records are held in its slot order from the start.
-// f32 rows of few values pay the counting pass for nothing: whole sort [64, 50257]
-// of ten values 147 us without bins and in whole chunks, 168 now ([64, 201088]
-// 360 / 302), of bf16 values held in f32 122 / 136 (327 / 290).
+// four workgroups to a CU: 994; in half chunks 1185, 1138 with one order of slots
+// throughout, which left no register spilled, 983 with the slots shared out
+// evenly).  bf16 keys, key ranges of few values and bunched keys pile up in the
+// bins and take the stable radix sort on the key; the records are held in its
+// slot order from the start.  f32 rows of few values pay the counting pass for
+// nothing: whole sort [64, 50257] of ten values 148 us without bins and in whole
+// chunks, 158 now ([64, 201088] 356 / 297), of bf16 values held in f32 122 / 125
+// (329 / 276).
 template <int NT, int E, int DT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(E <= 16 ? 4 : 2, 8)))
 void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs, const int32_t* table) {
@@ -555,8 +560,11 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs, const i
   const int n = s_off[R];  // at most CAP (the split's bound)
   if (n > CAP) return;     // never taken; keeps a broken table from writing past the LDS buffer
   const int64_t o0 = tp[(bp.K + 1) * R + k];
-  // a thread's slots, as the radix sort numbers them: ascending
-  auto slot_of = [&](int r) -> int { return w * (E * kWave) + r * kWave + l; };
+  // A thread's slots, as the radix sort numbers them: ascending, and shared out
+  // evenly where the bucket is not full (with 16 per thread, a bucket of a quarter
+  // lay in one wave: f32 [21, 40622] 61.0 -> 54.8 us, [1024, 201088] 2338 -> 2191).
+  const int per = (n + NT - 1) / NT;
+  auto slot_of = [&](int r) -> int { return r < per ? w * (per * kWave) + r * kWave + l : CAP; };
   uint64_t v[E];
   {
     // a row's records span less than 2^32 bytes: 32-bit offsets from its start
@@ -683,7 +691,7 @@ void bucket_sort_kernel(SortArgs a, BucketPlan bp, const uint64_t* runs, const i
       kor |= red[1][i];
     }
     // the low order bits of a bf16 key follow from the high
-    radix_sort_slots<E, NT>(v, buf, hist, wsum, (kand ^ kor) & (DT == kBF16 ? 0xFFFF0000u : ~0u), n);
+    radix_sort_slots<E, NT>(v, buf, hist, wsum, (kand ^ kor) & (DT == kBF16 ? 0xFFFF0000u : ~0u), n, per);
   }
   // outputs at o0 + rank: the source column, the sorted key and the gathered
   // second key (32-bit offsets from the bucket's first output)
